@@ -155,10 +155,10 @@ int sw_spmv_csr_f32(const int32_t *row_offsets, const int32_t *column_indices,
  * column_indices[nnz], values[nnz], vector[cols], output[rows]; entries in
  * any order, repeated coordinates add up.  The output is zeroed, then
  * accumulated.  Replaces ThreadPerNonzeroCOOSpMVPattern
- * (SparseWaveToGPU.cpp:154-214), which reads only spmv-block-size; with
- * spmv-mapping=wave-per-position a run-segmented kernel (one atomic per run
- * of equal adjacent rows, spmv-positions-per-lane entries per lane) is used
- * instead.
+ * (SparseWaveToGPU.cpp:154-214), which reads only spmv-block-size, by a
+ * run-segmented kernel: one atomic add per run of equal adjacent rows.  With
+ * spmv-mapping=wave-per-position each lane takes spmv-positions-per-lane
+ * entries; otherwise the library chooses.
  */
 int sw_spmv_coo_f32(const int32_t *row_indices, const int32_t *column_indices,
                     const float *values, const float *vector, float *output,

@@ -9,7 +9,7 @@
 //   thread-per-position SparsePositionScheduling.cpp:135-316
 //   wave-per-position  SparsePositionScheduling.cpp:318-403,
 //                      SparsePositionToSCF.cpp:190-271, SparseGPUUtils.cpp:247-292
-//   COO thread-per-nonzero SparseWaveToGPU.cpp:154-214
+//   COO SpMV           SparseWaveToGPU.cpp:154-214
 #include "sw_device.h"
 #include "sw_internal.h"
 
@@ -816,21 +816,9 @@ __global__ __launch_bounds__(256) void csr_row_at_position_kernel(
 // column-index and value arrays, entries in any order, coordinates may
 // repeat; the output is zeroed first, then accumulated.
 //
-// thread-per-nonzero: the reference's COO lowering
-// (ThreadPerNonzeroCOOSpMVPattern, SparseWaveToGPU.cpp:154-214), one thread
-// and one atomic add of val*x[col] per stored entry.
-__global__ __launch_bounds__(1024) void coo_thread_per_nonzero(
-    const int32_t *__restrict__ ri, const int32_t *__restrict__ col,
-    const float *__restrict__ val, const float *__restrict__ x,
-    float *__restrict__ y, int64_t nnz) {
-  const int64_t p = block_id() * blockDim.x + threadIdx.x;
-  if (p < nnz)
-    unsafeAtomicAdd(y + ld_nontemporal(ri + p),
-                    ld_nontemporal(val + p) * x[ld_nontemporal(col + p)]);
-}
-
-// Run-segmented COO (Wave64 extension, taken under the position mapping):
-// grid lane u takes entries [u*P, u*P+P).  Runs of equal adjacent row
+// Run-segmented COO, for every mapping (the reference's lowering,
+// ThreadPerNonzeroCOOSpMVPattern, SparseWaveToGPU.cpp:154-214, adds every
+// entry atomically): grid lane u takes entries [u*P, u*P+P).  Runs of equal adjacent row
 // indices are summed in registers; a run that closes inside the lane is added
 // atomically; the lane's last run is carried across lanes by a segmented scan
 // keyed on run numbers (a ballot prefix count of run starts, which is
@@ -1170,39 +1158,42 @@ int launch_spmv_coo(const int32_t *ri, const int32_t *col, const float *val,
   int rc = launch_fill_zero(y, rows, B, st);
   if (rc || nnz == 0)
     return rc;
-  if (streq(o.spmv_mapping, "wave-per-position")) {
-    const int64_t P = o.spmv_positions_per_lane;
-    const int64_t grid = std::max<int64_t>(ceil_div(ceil_div(nnz, P), B), 1);
-    rc = check_grid(grid, B, "run-segmented COO SpMV");
-    if (rc)
-      return rc;
-    const bool vec = aligned16(ri) && aligned16(col) && aligned16(val) &&
-                     narrow_offsets(cols, 1);
-    switch (P) {
-    case 1: launch_coo_runs<1, false>(grid, B, st, ri, col, val, x, y, nnz); break;
-    case 2: launch_coo_runs<2, false>(grid, B, st, ri, col, val, x, y, nnz); break;
-    case 4:
-      if (vec) launch_coo_runs<4, true>(grid, B, st, ri, col, val, x, y, nnz);
-      else launch_coo_runs<4, false>(grid, B, st, ri, col, val, x, y, nnz);
-      break;
-    case 8:
-      if (vec) launch_coo_runs<8, true>(grid, B, st, ri, col, val, x, y, nnz);
-      else launch_coo_runs<8, false>(grid, B, st, ri, col, val, x, y, nnz);
-      break;
-    default:
-      if (vec) launch_coo_runs<16, true>(grid, B, st, ri, col, val, x, y, nnz);
-      else launch_coo_runs<16, false>(grid, B, st, ri, col, val, x, y, nnz);
-      break;
-    }
-    return launch_check("run-segmented COO SpMV kernel");
-  }
-  const int64_t grid = std::max<int64_t>(ceil_div(nnz, B), 1);
-  rc = check_grid(grid, B, "thread-per-nonzero COO SpMV");
+  const bool vec = aligned16(ri) && aligned16(col) && aligned16(val) &&
+                   narrow_offsets(cols, 1);
+  // The position mapping gives P; the others leave it to the kernel: four
+  // entries per lane in 128-bit loads where the arrays allow it, else one
+  // (4-byte loads of consecutive lanes are coalesced only at P = 1).  Row-
+  // sorted entries, 300,007 rows of 16 on average: P = 1 / 2 / 4 / 8 32 /
+  // 39 / 32 / 32 us, 1,000,000 rows of 20: 131 / 160 / 128 / 130 us, against
+  // 300 and 1235 us with one thread and one atomic add per entry; shuffled
+  // entries (every run one entry) 250 and 981 us either way.
+  const int64_t P = streq(o.spmv_mapping, "wave-per-position")
+                        ? o.spmv_positions_per_lane
+                        : (vec ? 4 : 1);
+  // whole waves (spmv-block-size may be any size outside the position
+  // mapping)
+  const int64_t RB = ceil_div(B, kWave) * kWave;
+  const int64_t grid = std::max<int64_t>(ceil_div(ceil_div(nnz, P), RB), 1);
+  rc = check_grid(grid, RB, "run-segmented COO SpMV");
   if (rc)
     return rc;
-  hipLaunchKernelGGL(coo_thread_per_nonzero, grid_dim(grid, B),
-                     dim3((unsigned)B), 0, st, ri, col, val, x, y, nnz);
-  return launch_check("thread-per-nonzero COO SpMV kernel");
+  switch (P) {
+  case 1: launch_coo_runs<1, false>(grid, RB, st, ri, col, val, x, y, nnz); break;
+  case 2: launch_coo_runs<2, false>(grid, RB, st, ri, col, val, x, y, nnz); break;
+  case 4:
+    if (vec) launch_coo_runs<4, true>(grid, RB, st, ri, col, val, x, y, nnz);
+    else launch_coo_runs<4, false>(grid, RB, st, ri, col, val, x, y, nnz);
+    break;
+  case 8:
+    if (vec) launch_coo_runs<8, true>(grid, RB, st, ri, col, val, x, y, nnz);
+    else launch_coo_runs<8, false>(grid, RB, st, ri, col, val, x, y, nnz);
+    break;
+  default:
+    if (vec) launch_coo_runs<16, true>(grid, RB, st, ri, col, val, x, y, nnz);
+    else launch_coo_runs<16, false>(grid, RB, st, ri, col, val, x, y, nnz);
+    break;
+  }
+  return launch_check("run-segmented COO SpMV kernel");
 }
 
 } // namespace sw

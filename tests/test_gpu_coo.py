@@ -15,7 +15,7 @@ from tests._check import assert_within_bound
 pytestmark = pytest.mark.gpu
 
 MAPPINGS = [
-    "",  # reference lowering: thread per nonzero, spmv-block-size 256
+    "",  # no mapping: the run length is the library's choice
     "spmv-block-size=64",
     "spmv-mapping=wave-per-position spmv-positions-per-lane=1",
     "spmv-mapping=wave-per-position spmv-positions-per-lane=4",
@@ -160,3 +160,17 @@ def test_reference_sweep_matrices(dev, workload):
     for opts in MAPPINGS:
         np.testing.assert_array_equal(_run(csr.rows, ri, ci, val, x, opts),
                                       want, err_msg=opts)
+
+
+@pytest.mark.parametrize("block", [1, 100, 256, 1000])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("n", [1, 255, 257, 1025, 70001])
+def test_default_mapping_block_sizes(dev, orc, block, offset, n):
+    """Without a mapping any spmv-block-size runs as whole waves: aligned
+    arrays four entries per lane, others (offset 1) one."""
+    rng = np.random.default_rng(n + block)
+    ri = np.sort(rng.integers(0, 300, n)).astype(np.int32)
+    ci = rng.integers(0, 200, n).astype(np.int32)
+    val = rng.uniform(-1, 1, n).astype(np.float32)
+    x = rng.uniform(-1, 1, 200).astype(np.float32)
+    _check(orc, 300, ri, ci, val, x, f"spmv-block-size={block}", offset)
