@@ -25,8 +25,8 @@
  * (larger: SW_ERR_INVALID_SHAPE before any launch); COO takes any nnz.
  * Every mapping runs at those limits: a launch of more than 2^32 - 1
  * work-items, which one grid dimension cannot hold, is folded into a 2-D
- * grid, and the BSR SpMM past about 8.4 million block rows computes with
- * its thread-per-output kernel.
+ * grid, and a BSR SpMM whose block rows one grid dimension cannot hold
+ * (past about 8.4 million) computes with its thread-per-output kernel.
  *
  * Citations are path:line into the reference (sott0n/SparseWaveComp).
  */
@@ -240,8 +240,8 @@ int sw_bsr_spmm_bf16_f32out(const int32_t *block_row_offsets,
 /*
  * BSR slab floor, a diagnostic with no counterpart in the reference: the
  * launch that sw_bsr_spmm_f32 / _bf16 / _bf16_f32out make on the matrix
- * cores for these operands (16 x 16 blocks; value_bytes 4 with k % 4 == 0,
- * or 2 with k % 8 == 0; 16-byte aligned rhs and output; output_bytes 4, or 2
+ * cores for these operands with 64 < k <= 128 (16 x 16 blocks; value_bytes 4
+ * with k % 4 == 0, or 2 with k % 8 == 0; other k run that kernel's strips; 16-byte aligned rhs and output; output_bytes 4, or 2
  * for the bf16 output) with its grid, block order, block and RHS-slab
  * loads, LDS reduction and stores unchanged and the block products replaced
  * by an XOR of the 32-bit words each lane loads.  Every output element of a

@@ -5,22 +5,21 @@
 // row-major [nnzb][b][b] (SparseWaveOps.td:133-137), shape rules of the
 // verifier (lib/Dialect/SparseWave/IR/SparseWaveOps.cpp:144-207, 340-372).
 //
-// The MI355X path for 16 x 16 blocks runs each block product on the matrix
-// cores, accumulating in fp32 registers across the block row's blocks:
+// The MI355X path runs each block product on the matrix cores, accumulating
+// in fp32 registers across the block row's blocks; for 16 x 16 blocks:
 //   fp32, k % 4 == 0: a wave owns a 16 x 64 output strip (four tiles with
 //     interleaved columns, 128-bit RHS loads and output stores) and issues
 //     v_mfma_f32_16x16x4_f32 four times per block and tile;
 //   bf16 with a bf16 output, k % 8 == 0: a wave owns a 16 x 128 output strip
 //     (eight tiles with interleaved columns, 128-bit RHS loads) and issues
 //     v_mfma_f32_16x16x16_bf16 once per block and tile;
-//   otherwise a workgroup of four waves owns one block row and 128 output
-//     columns, each wave two 16 x 16 tiles, issuing
-//     fp32: v_mfma_f32_16x16x4_f32 four times per block and tile,
-//     bf16: v_mfma_f32_16x16x16_bf16 once per block and tile.
+//   other block sizes that are a multiple of 4, other k and unaligned
+//     operands take bsr_mfma, the same tiles over 16-row strips.
 #include "sw_device.h"
 #include "sw_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace swd;
 
@@ -83,124 +82,6 @@ __device__ __forceinline__ int xcd_block_row(int w, int nbr) {
   if (nbr % kXcds != 0)
     return w;
   return (w % kXcds) * (nbr / kXcds) + w / kXcds;
-}
-
-// Blocks are processed in batches of NB: the batch's column indices arrive
-// with one load (lane j holds block j's column, broadcast by v_readlane),
-// then every A and B operand of the batch is requested before the first
-// MFMA, so a block row waits for two memory latencies per batch instead of
-// two per block.
-template <int NB>
-__global__ __launch_bounds__(256) void bsr16_mfma_f32(
-    const int32_t *__restrict__ bro, const int32_t *__restrict__ bcol,
-    const float *__restrict__ bval, const float *__restrict__ rhs,
-    float *__restrict__ out, int64_t k, int nbr) {
-  const int br = xcd_block_row(blockIdx.x, nbr);
-  const int wave = wave_in_group();
-  const int l = lane_id();
-  const int i = l & 15, g = l >> 4;
-  const int64_t n0 = (int64_t)blockIdx.y * 128 + wave * 32;
-  const int64_t c0 = n0 + i, c1 = n0 + 16 + i;
-  const bool ok0 = c0 < k, ok1 = c1 < k;
-  v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  const int32_t s = bro[br], e = bro[br + 1];
-  for (int32_t b0 = s; b0 < e; b0 += NB) {
-    const int nb = e - b0 < NB ? e - b0 : NB; // wave-uniform
-    const int bcl = l < nb ? bcol[b0 + l] : 0;
-    v4f a[NB];
-    float bv0[NB][4], bv1[NB][4];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      if (j < nb) {
-        const int64_t bc = __builtin_amdgcn_readlane(bcl, j);
-        a[j] = ld_stream(reinterpret_cast<const v4f *>(
-            bval + (int64_t)(b0 + j) * 256 + i * 16 + g * 4));
-        const float *brow = rhs + (bc * 16 + g * 4) * k;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          bv0[j][st] = ok0 ? brow[st * k + c0] : 0.0f;
-          bv1[j][st] = ok1 ? brow[st * k + c1] : 0.0f;
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      if (j < nb) {
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][st], bv0[j][st],
-                                                      acc0, 0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][st], bv1[j][st],
-                                                      acc1, 0, 0, 0);
-        }
-      }
-    }
-  }
-  // non-temporal stores: the output is not re-read, so it should not
-  // displace RHS tiles from the caches
-  float *o = out + ((int64_t)br * 16 + g * 4) * k;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    if (ok0)
-      __builtin_nontemporal_store(acc0[v], o + v * k + c0);
-    if (ok1)
-      __builtin_nontemporal_store(acc1[v], o + v * k + c1);
-  }
-}
-
-template <int NB, typename TO>
-__global__ __launch_bounds__(256) void bsr16_mfma_bf16(
-    const int32_t *__restrict__ bro, const int32_t *__restrict__ bcol,
-    const uint16_t *__restrict__ bval, const uint16_t *__restrict__ rhs,
-    TO *__restrict__ out, int64_t k, int nbr) {
-  const int br = xcd_block_row(blockIdx.x, nbr);
-  const int wave = wave_in_group();
-  const int l = lane_id();
-  const int i = l & 15, g = l >> 4;
-  const int64_t n0 = (int64_t)blockIdx.y * 128 + wave * 32;
-  const int64_t c0 = n0 + i, c1 = n0 + 16 + i;
-  const bool ok0 = c0 < k, ok1 = c1 < k;
-  v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  const int32_t s = bro[br], e = bro[br + 1];
-  for (int32_t b0 = s; b0 < e; b0 += NB) {
-    const int nb = e - b0 < NB ? e - b0 : NB;
-    const int bcl = l < nb ? bcol[b0 + l] : 0;
-    v4s a[NB], bv0[NB], bv1[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      if (j < nb) {
-        const int64_t bc = __builtin_amdgcn_readlane(bcl, j);
-        // A[i][4g .. 4g+3]: 8 contiguous bytes of the row-major block
-        a[j] = *reinterpret_cast<const v4s *>(bval + (int64_t)(b0 + j) * 256 +
-                                              i * 16 + g * 4);
-        const uint16_t *brow = rhs + (bc * 16 + g * 4) * k;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          bv0[j][st] = ok0 ? (short)brow[st * k + c0] : (short)0;
-          bv1[j][st] = ok1 ? (short)brow[st * k + c1] : (short)0;
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      if (j < nb) {
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j], bv0[j], acc0, 0,
-                                                         0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j], bv1[j], acc1, 0,
-                                                         0, 0);
-      }
-    }
-  }
-  // non-temporal stores: the output is not re-read, so it should not
-  // displace RHS tiles from the caches
-  TO *o = out + ((int64_t)br * 16 + g * 4) * k;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    if (ok0)
-      st1_nt(o + v * k + c0, acc0[v]);
-    if (ok1)
-      st1_nt(o + v * k + c1, acc1[v]);
-  }
 }
 
 // Column-interleaved bf16 kernel (k % 8 == 0, rhs and output 16-byte
@@ -483,6 +364,222 @@ __global__ __launch_bounds__(64 * kF32Strips * SPL) void bsr16_mfma_f32_x4(
   }
 }
 
+// Matrix-core kernel for any block size that is a multiple of 4 and any k,
+// fp32 and bf16 (16 x 16 blocks with aligned operands take the two kernels
+// above, whose blocks are wave-uniform).
+//
+// A block row's blocks side by side are a b x (blocks b) matrix, whose
+// columns ("virtual k") are taken 16 at a time: lane group g of a wave holds
+// virtual k 16 v + 4 g .. + 3 of step v, four columns of one block since b
+// is a multiple of 4 -- so 4 x 4 blocks go four to a step, 8 x 8 two, and a
+// 32 x 32 block takes two steps.  Each lane tracks its own (block, column)
+// and loads that block's rhs rows itself, N = 16 bytes' worth of consecutive
+// output columns each: one 128-bit load of an rhs row gives a lane its
+// values for N interleaved 16-column tiles, as in the kernels above.  Output
+// rows are taken MS 16-row strips at a time, which share those rhs loads; a
+// workgroup owns one group of MS strips of one block row and 16 N columns,
+// and its SPL waves split the steps (wave w takes w, w + SPL, ...), the
+// partial tiles summed through LDS.  Steps past the block row's end load
+// nothing and multiply zeros; D rows past b are not stored.
+//
+// It is bound by the rhs slabs' trips from L2 and the MALL.  2,048 block
+// rows of 32 x 32 blocks (9.25 on average), bf16, 200 columns: 1966 us for
+// the thread-per-output loop, 34.5 us here (242 MB of slabs, 7 TB/s).
+//
+// VEC: block values aligned to four elements, rhs and output to 16 bytes
+// and k a multiple of N, so that every access is aligned and no lane's
+// columns pass k.  Otherwise the same accesses are element-aligned, and a
+// lane whose columns pass k reads on into the next row (columns of B are
+// independent, and those past k are not stored); a step that could so read
+// past the end of rhs (total elements) loads element by element.
+template <typename T, typename TO, int MS, int N, int SPL, bool VEC>
+__global__ __launch_bounds__(64 * SPL, 4) void bsr_mfma(
+    const int32_t *__restrict__ bro, const int32_t *__restrict__ bcol,
+    const T *__restrict__ bval, const T *__restrict__ rhs,
+    TO *__restrict__ out, int64_t k, int32_t b, int32_t groups,
+    int32_t strips, int64_t total) {
+  constexpr bool kF32 = sizeof(T) == 4;
+  using AV = std::conditional_t<kF32, v4f, v2u>; // four A values
+  // N rhs values: a lane's columns, one per tile
+  using BV = std::conditional_t<kF32, v4f, std::conditional_t<N == 8, v4u, v2u>>;
+  __shared__ v4f red[SPL > 1 ? SPL - 1 : 1][MS][N][kWave];
+  // (gridDim.x < 2^32 / 256)
+  const uint32_t id = (uint32_t)xcd_contiguous(blockIdx.x, gridDim.x);
+  const uint32_t vb = id / (uint32_t)strips;
+  const int32_t br = (int32_t)(vb / (uint32_t)groups);
+  const int32_t s0 = 16 * MS * (int32_t)(vb - (uint32_t)br * groups);
+  const int sp = wave_in_group();
+  const int l = lane_id(), i = l & 15, g = l >> 4;
+  // column strips in x, fastest, so that a block row's strips share its blocks
+  // and the rhs lines between them in one XCD's L2 (strips = 1: in y)
+  const int64_t cb =
+      ((int64_t)blockIdx.y + (id - vb * (uint32_t)strips)) * (16 * N) + N * i;
+  const bool ok = cb < k;
+  v4f acc[MS][N];
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+      acc[m][t] = v4f{0.f, 0.f, 0.f, 0.f};
+  const int32_t s = bro[br], n = bro[br + 1] - s;
+  // the lane's first virtual k and the advance of SPL steps
+  int32_t blk = (16 * sp + 4 * g) / b;
+  int32_t r = 16 * sp + 4 * g - blk * b;
+  const int32_t dblk = 16 * SPL / b, dr = 16 * SPL - dblk * b;
+  // a step's operands: its A rows and the rhs rows of block column c
+  // (zeros past the block row's end); moves the lane to the next step
+  auto load = [&](int32_t c, AV (&a)[MS], BV (&q)[4])
+      __attribute__((always_inline)) {
+    const bool in = blk < n, live = ok && in;
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+      a[m] = AV{};
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+      q[st] = BV{};
+    const int64_t at = ((int64_t)c * b + r) * k + cb;
+    bool whole = true; // no lane's rhs loads pass the end of rhs
+    if constexpr (!VEC)
+      whole = __builtin_amdgcn_ballot_w64(live && at + 3 * k + N > total) == 0;
+    if (in) {
+      const T *ap = bval + (int64_t)(s + blk) * b * b + r;
+#pragma unroll
+      for (int m = 0; m < MS; ++m) {
+        const T *av = ap + (int64_t)std::min(s0 + 16 * m + i, b - 1) * b;
+        if constexpr (VEC)
+          a[m] = ld_stream(reinterpret_cast<const AV *>(av));
+        else
+          __builtin_memcpy(&a[m], av, sizeof(AV));
+      }
+    }
+    if (whole) { // wave-uniform
+      if (live) {
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          if constexpr (VEC)
+            q[st] = *reinterpret_cast<const BV *>(rhs + at + st * k);
+          else
+            __builtin_memcpy(&q[st], rhs + at + st * k, sizeof(BV));
+        }
+      }
+    } else if (live) {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        T x[N];
+#pragma unroll
+        for (int t = 0; t < N; ++t)
+          x[t] = cb + t < k ? rhs[at + st * k + t] : T(0);
+        __builtin_memcpy(&q[st], x, sizeof(BV));
+      }
+    }
+    r += dr;
+    blk += dblk;
+    if (r >= b) {
+      r -= b;
+      ++blk;
+    }
+  };
+  // a step's block column, loaded a step ahead
+  auto column = [&](int32_t at) __attribute__((always_inline)) {
+    return bcol[s + std::min(at, n - 1)];
+  };
+  auto products = [&](const AV (&a)[MS], const BV (&q)[4])
+      __attribute__((always_inline)) {
+    if constexpr (kF32) {
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int t = 0; t < N; ++t)
+#pragma unroll
+          for (int m = 0; m < MS; ++m)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                a[m][st], q[st][t], acc[m][t], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < N; ++t) {
+        // element t of the four rows, paired by byte permutes
+        const int d = t >> 1;
+        const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
+        const v2u bt = v2u{__builtin_amdgcn_perm(q[1][d], q[0][d], sel),
+                           __builtin_amdgcn_perm(q[3][d], q[2][d], sel)};
+#pragma unroll
+        for (int m = 0; m < MS; ++m)
+          acc[m][t] = mfma_16x16x16_bf16(a[m], bt, acc[m][t]);
+      }
+    }
+  };
+  // this wave's steps (a loop that tested lane 0's block instead copied
+  // every accumulator in each step; a step's operands requested a whole
+  // step ahead, two buffers, measured no faster)
+  const int64_t steps = ((int64_t)n * b + 15) / 16;
+  const int32_t mine = (int32_t)((steps - sp + SPL - 1) / SPL);
+  int32_t c = mine > 0 ? column(blk) : 0;
+  for (int32_t t = 0; t < mine; ++t) {
+    const int32_t next = column(blk + dblk + (r + dr >= b ? 1 : 0));
+    AV a[MS];
+    BV q[4];
+    load(c, a, q);
+    products(a, q);
+    c = next;
+  }
+  // wave m % SPL sums and stores strip m
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+    if (sp != m % SPL)
+#pragma unroll
+      for (int t = 0; t < N; ++t)
+        red[sp < m % SPL ? sp : sp - 1][m][t][l] = acc[m][t];
+  __syncthreads();
+  if (!ok)
+    return; // after the only barrier
+#pragma unroll
+  for (int m = 0; m < MS; ++m) {
+    if (sp != m % SPL) // wave-uniform
+      continue;
+#pragma unroll
+    for (int w = 0; w < SPL - 1; ++w)
+#pragma unroll
+      for (int t = 0; t < N; ++t)
+        acc[m][t] += red[w][m][t][l];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int32_t row = s0 + 16 * m + 4 * g + v;
+      if (row >= b)
+        continue;
+      TO *o = out + ((int64_t)br * b + row) * k + cb;
+      if (VEC || cb + N <= k) {
+        if constexpr (sizeof(TO) == 2) {
+          uint32_t y[N / 2];
+#pragma unroll
+          for (int t = 0; t < N; t += 2)
+            y[t / 2] = pack_bf16x2(acc[m][t][v], acc[m][t + 1][v]);
+          BV z;
+          __builtin_memcpy(&z, y, sizeof z);
+          if constexpr (VEC)
+            __builtin_nontemporal_store(z, reinterpret_cast<BV *>(o));
+          else
+            __builtin_memcpy(o, &z, sizeof z);
+        } else {
+#pragma unroll
+          for (int t = 0; t < N; t += 4) {
+            const v4f y = v4f{acc[m][t][v], acc[m][t + 1][v],
+                              acc[m][t + 2][v], acc[m][t + 3][v]};
+            if constexpr (VEC)
+              st4_nt(o + t, y);
+            else
+              __builtin_memcpy(o + t, &y, sizeof y);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < N; ++t)
+          if (cb + t < k)
+            stv(o + t, acc[m][t][v]);
+      }
+    }
+  }
+}
+
 // fp32 x4 kernel shape: blocks per batch and waves per strip. Configuration
 // 4, two strips per workgroup: 1 wave x 4-block batches 134.0 us, 2 x 2
 // 127.5 us, 2 x 1 128.3 us, 2 x 4 144.2 us, 4 x 2 130.3 us, 4 x 1 124.0 us.
@@ -526,73 +623,99 @@ constexpr int kBf16Split = 4;
 
 template <typename T, typename TO>
 int launch_bsr(const int32_t *bro, const int32_t *bcol, const T *bval,
-               const T *rhs, TO *out, int64_t rows, int64_t nnzb, int64_t k,
-               int64_t b, const sw_options &o, hipStream_t st, bool mfma_ok) {
-  (void)nnzb;
+               const T *rhs, TO *out, int64_t rows, int64_t cols, int64_t k,
+               int64_t b, const sw_options &o, hipStream_t st, bool mfma) {
   if (rows == 0 || k == 0)
     return SW_OK;
   const int nbr = (int)(rows / 16);
-  // The matrix-core kernels index block rows by blockIdx.x alone (y holds
-  // the column strips), so their x must stay within one grid dimension's
-  // 2^32 - 1 work-items (512-work-item workgroups: about 8.4 million block
-  // rows); past it the thread-per-output kernel below, whose launch folds,
-  // computes the product.
-  mfma_ok = mfma_ok && nbr <= sw::grid_row(512);
+  // The matrix-core kernels' x must stay within one grid dimension's
+  // 2^32 - 1 work-items; past it the thread-per-output kernel below, whose
+  // launch folds, computes the product.
+  const bool b16 = mfma && b == 16 && rows / 16 <= sw::grid_row(512) &&
+                   (reinterpret_cast<uintptr_t>(bval) &
+                    (4 * sizeof(T) - 1)) == 0;
+  if (b16 && k > (int64_t)65535 * 128)
+    return sw::fail(SW_ERR_INVALID_SHAPE, "rhs has too many columns");
+  // The kernels for 16 x 16 blocks whose values are aligned to four elements
+  // (they read A rows as 16-byte (fp32) or 8-byte (bf16) vectors) take 64 <
+  // k <= 128; on both sides of that bsr_mfma is faster (us, fp32 k = 64
+  // 68.9 against 66.0 us, k = 128 125.5 / 126.7, k = 256 289 / 266; bf16
+  // k = 64 53 / 38, k = 128 57.4 / 55.6, k = 200 118 / 94: a narrow strip
+  // leaves most of their lanes idle, and their strips of one block row lie
+  // a whole grid apart)
+  const bool mfma_ok = b16 && k > 64 && k <= 128;
   if constexpr (sizeof(T) == 4) {
-    // fp32 with k % 4 == 0 takes the column-interleaved kernel (measured on
-    // configuration 4: 167 us against 189 us for the one-column-per-lane
-    // kernel below, before the block row was split over waves)
+    // fp32 with k % 4 == 0 takes the column-interleaved kernel
     if (mfma_ok && k % 4 == 0 && sw::aligned16(rhs) && sw::aligned16(out)) {
-      const int64_t strips =
-          std::min<int64_t>(kF32Strips, sw::ceil_div(k, 64));
-      const int64_t gy = sw::ceil_div(k, 64 * strips);
-      if (gy > 65535)
-        return sw::fail(SW_ERR_INVALID_SHAPE, "rhs has too many columns");
-      const int rc = sw::check_flat_grid(nbr, 64 * strips * kF32Split,
-                                         "BSR MFMA kernel");
-      if (rc)
-        return rc;
       hipLaunchKernelGGL((bsr16_mfma_f32_x4<kF32Batch, kF32Split>),
-                         dim3((unsigned)nbr, (unsigned)gy),
-                         dim3((unsigned)(64 * strips * kF32Split)), 0, st, bro,
-                         bcol, bval, rhs, out, k, nbr);
+                         dim3((unsigned)nbr), dim3(64 * kF32Strips * kF32Split),
+                         0, st, bro, bcol, bval, rhs, out, k, nbr);
       return sw::launch_check("BSR MFMA kernel");
     }
   } else {
     // k % 8 == 0: eight interleaved tiles per workgroup, 128-bit RHS loads
-    // (configuration 4: bf16 output 57.1 us against 69.8 us for the two-tile
-    // kernel below; fp32 output 74.3 against 73.7 us)
-    {
-      if (mfma_ok && k % 8 == 0 && sw::aligned16(rhs) && sw::aligned16(out)) {
-        const int64_t gy = sw::ceil_div(k, 128);
-        if (gy > 65535)
-          return sw::fail(SW_ERR_INVALID_SHAPE, "rhs has too many columns");
-        const int rc =
-            sw::check_flat_grid(nbr, 64 * kBf16Split, "BSR MFMA kernel");
-        if (rc)
-          return rc;
-        hipLaunchKernelGGL((bsr16_mfma_bf16_x8<kBf16Batch, kBf16Split, TO>),
-                           dim3((unsigned)nbr, (unsigned)gy),
-                           dim3(64 * kBf16Split), 0, st, bro, bcol, bval,
-                           rhs, out, k, nbr);
-        return sw::launch_check("BSR MFMA kernel");
-      }
+    if (mfma_ok && k % 8 == 0 && sw::aligned16(rhs) && sw::aligned16(out)) {
+      hipLaunchKernelGGL((bsr16_mfma_bf16_x8<kBf16Batch, kBf16Split, TO>),
+                         dim3((unsigned)nbr), dim3(64 * kBf16Split), 0, st, bro,
+                         bcol, bval, rhs, out, k, nbr);
+      return sw::launch_check("BSR MFMA kernel");
     }
   }
-  if (mfma_ok) {
-    int64_t gy = sw::ceil_div(k, 128);
-    if (gy > 65535)
-      return sw::fail(SW_ERR_INVALID_SHAPE, "rhs has too many columns");
-    const int rc = sw::check_flat_grid(nbr, 256, "BSR MFMA kernel");
-    if (rc)
-      return rc;
-    dim3 grid((unsigned)nbr, (unsigned)gy);
-    if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL(bsr16_mfma_f32<8>, grid, dim3(256), 0, st, bro, bcol,
-                         bval, rhs, out, k, nbr);
-    else
-      hipLaunchKernelGGL((bsr16_mfma_bf16<8, TO>), grid, dim3(256), 0, st, bro,
-                         bcol, bval, rhs, out, k, nbr);
+  // Every other shape with b a multiple of 4; a launch that one grid
+  // dimension cannot hold takes the thread-per-output kernel below.  Sweeps
+  // (us, mean blocks per block row in parentheses):
+  // * bf16, waves per strip group 1 / 2 / 4: 32 x 32 blocks, 2,048 block
+  //   rows (9.25), k = 200 41.1 / 34.5 / 40.2; k = 64 (columns per lane 4)
+  //   20.7 / 15.4 / 17.8; 16 x 16, 16,384 block rows (8), k = 200 122.9 /
+  //   93.7 / 97.0, k = 30 29.5 / 29.4 / 33.5.
+  // * bf16, columns per lane 8 / 4: k = 61 44.2 / 38.6, k = 100 47.8 / 82.4
+  //   (two strips): 4 where one strip of 64 columns holds k.
+  // * fp32, 2 / 4 waves: 32 x 32, k = 200 137.7 / 127.2; 16 x 16, k = 256
+  //   268.7 / 266.2; 8 x 8 (half the steps), k = 45 31.8 / 35.4.
+  const int64_t N = sizeof(T) == 2 && k > 64 ? 8 : 4;
+  const int64_t SPL = sizeof(T) == 2 || b < 16 ? 2 : 4;
+  const int64_t gy = sw::ceil_div(k, 16 * N);
+  const int64_t groups = sw::ceil_div(b, 32);
+  const int64_t x = rows / b * groups, row = sw::grid_row(64 * SPL);
+  if (mfma && b % 4 == 0 && b <= (1 << 24) && x <= row &&
+      (gy <= 65535 || gy <= row / x)) {
+    // one grid dimension where it holds them all
+    const int64_t strips = gy <= row / x ? gy : 1;
+    const bool vec = k % N == 0 && sw::aligned16(rhs) && sw::aligned16(out) &&
+                     (reinterpret_cast<uintptr_t>(bval) &
+                      (4 * sizeof(T) - 1)) == 0;
+    const dim3 grid((unsigned)(x * strips), (unsigned)(gy / strips));
+#define SW_BSR_ANY(MS, N, SPL)                                                \
+  do {                                                                        \
+    if (vec)                                                                  \
+      hipLaunchKernelGGL((bsr_mfma<T, TO, MS, N, SPL, true>), grid,           \
+                         dim3(64 * SPL), 0, st, bro, bcol, bval, rhs, out, k, \
+                         (int32_t)b, (int32_t)groups, (int32_t)strips,        \
+                         cols * k);                                           \
+    else                                                                      \
+      hipLaunchKernelGGL((bsr_mfma<T, TO, MS, N, SPL, false>), grid,          \
+                         dim3(64 * SPL), 0, st, bro, bcol, bval, rhs, out, k, \
+                         (int32_t)b, (int32_t)groups, (int32_t)strips,        \
+                         cols * k);                                           \
+  } while (0)
+    if constexpr (sizeof(T) == 4) {
+      if (b > 16)
+        SW_BSR_ANY(2, 4, 4);
+      else if (b == 16)
+        SW_BSR_ANY(1, 4, 4);
+      else
+        SW_BSR_ANY(1, 4, 2);
+    } else {
+      if (b > 16 && N == 8)
+        SW_BSR_ANY(2, 8, 2);
+      else if (b > 16)
+        SW_BSR_ANY(2, 4, 2);
+      else if (N == 8)
+        SW_BSR_ANY(1, 8, 2);
+      else
+        SW_BSR_ANY(1, 4, 2);
+    }
+#undef SW_BSR_ANY
     return sw::launch_check("BSR MFMA kernel");
   }
   const int64_t B = o.spmm_block_size;
@@ -600,16 +723,16 @@ int launch_bsr(const int32_t *bro, const int32_t *bcol, const T *bval,
   int rc = sw::check_grid(grid, B, "BSR SpMM");
   if (rc)
     return rc;
-  const bool row = k % 64 == 0 && B % 64 == 0 && rows <= INT32_MAX;
+  const bool by_row = k % 64 == 0 && B % 64 == 0 && rows <= INT32_MAX;
 #define SW_BSR_TPO(BS, ROW)                                                   \
   hipLaunchKernelGGL((bsr_thread_per_output<T, TO, BS, ROW>),                 \
                      sw::grid_dim(grid, B), dim3((unsigned)B), 0, st, bro,   \
                      bcol, bval, rhs, out, rows, k, (int32_t)b)
-  if (b == 16 && row)
+  if (b == 16 && by_row)
     SW_BSR_TPO(16, true);
   else if (b == 16)
     SW_BSR_TPO(16, false);
-  else if (row)
+  else if (by_row)
     SW_BSR_TPO(0, true);
   else
     SW_BSR_TPO(0, false);
@@ -637,14 +760,10 @@ int bsr_entry(const int32_t *block_row_offsets,
     rc = sw::check_value_alignment(sizeof(TO), {output});
   if (rc)
     return rc;
-  // the MFMA kernels read A rows of a block as 16-byte (fp32) or 8-byte
-  // (bf16) vectors
-  const bool mfma = o.bsr_use_mfma && block_size == 16 &&
-                    (reinterpret_cast<uintptr_t>(block_values) &
-                     (4 * sizeof(T) - 1)) == 0;
   return launch_bsr<T, TO>(block_row_offsets, block_column_indices,
-                           block_values, rhs, output, rows, nnzb, k,
-                           block_size, o, sw::as_stream(stream), mfma);
+                           block_values, rhs, output, rows, cols, k,
+                           block_size, o, sw::as_stream(stream),
+                           o.bsr_use_mfma != 0);
 }
 
 // The slab floor: the MFMA kernel launch_bsr would run for these operands,

@@ -431,8 +431,8 @@ def _bsr_bf16(bsr, rhs, opts, out_dtype):
 @pytest.mark.parametrize("k", [128, 40, 200, 8, 30])
 @pytest.mark.parametrize("out_dtype", [BF, torch.float32])
 def test_bf16_bsr(dev, orc, opts, k, out_dtype):
-    """k % 8 == 0 takes the column-interleaved kernel (partial strips at 40
-    and 200); other k the scalar-load kernel."""
+    """64 < k <= 128 with k % 8 == 0 takes the 16 x 16 kernel, other k the
+    any-block-size kernel (partial strips at 40 and 200)."""
     bsr = W.bsr_banded(seed=k, rows=16 * 96, block_size=16, blocks_per_row=6,
                        band=3, band_blocks=3, value_std=0.5)
     rhs = np.random.default_rng(k).standard_normal((bsr.cols, k)).astype(

@@ -43,8 +43,8 @@ def test_bsr_golden(dev, golden, opts):
 
 
 @pytest.mark.parametrize("opts", BSR_OPTS)
-# k % 4 == 0 takes the column-interleaved MFMA kernels (partial strips at 40
-# and 200), other k the scalar-load MFMA kernels
+# b = 16 with 64 < k <= 128 and k % 4 == 0 takes the 16 x 16 kernel, the
+# others the any-block-size kernel (partial strips at 40 and 200)
 @pytest.mark.parametrize("b,k", [(16, 128), (16, 40), (16, 200), (16, 30),
                                  (16, 7), (4, 9), (4, 64), (8, 128)])
 def test_bsr_fp32(dev, orc, opts, b, k):
