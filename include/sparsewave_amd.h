@@ -346,6 +346,12 @@ int sw_csr_rowwise_map_bf16(const int32_t *row_offsets,
  * ten-buffer ABI (tools/sparsewave-bundle/sparsewave_bundle_ir.py:82-93):
  * query[rows][d], transposed_key[d][cols], value[cols][dv],
  * scores[nnz], row_maximum[rows], row_sum[rows], output[rows][dv].
+ * With sddmm-mapping=row-tile-mfma sddmm-lanes-per-row=64
+ * spmm-mapping=row-tile-mfma, and with every mapping and block size left at
+ * its default, one kernel runs the chain over 16-row tiles (d in {64, 128},
+ * dv % 16 == 0, nnz >= 4; without options also no output sharing memory
+ * with another buffer, the exponentials and divisions then as the separate
+ * ops compute them); other calls launch the separate ops.
  */
 int sw_sparse_attention_f32(const int32_t *row_offsets,
                             const int32_t *column_indices,

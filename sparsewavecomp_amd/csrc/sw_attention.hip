@@ -591,6 +591,473 @@ __device__ __forceinline__ void attention_row_softmax(
   }
 }
 
+// the eight K^T values K^T[32 s + 8 g + e][c] (e = 0..7) as four bf16 pairs;
+// base is K^T row 32 s, lane_off the byte offset of column c plus 8 g rows
+__device__ __forceinline__ v4u gather_kt8(const uint16_t *base,
+                                          uint32_t row_bytes,
+                                          uint32_t lane_off) {
+  uint32_t x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    x[e] = *at_bytes(at_bytes(base, e * row_bytes), lane_off);
+  return v4u{x[0] | (x[1] << 16), x[2] | (x[3] << 16), x[4] | (x[5] << 16),
+             x[6] | (x[7] << 16)};
+}
+
+// exp and division of the fused tiles.  LIBM: the library's expf and the
+// IEEE division, as the six separate ops compute them; otherwise the hardware
+// base-2 exponential (exp_by_exp2) and a multiply by the row's reciprocal.
+template <bool LIBM>
+__device__ __forceinline__ float tile_exp(float x) {
+  if constexpr (LIBM)
+    return expf(x);
+  else
+    return exp_by_exp2(x);
+}
+template <bool LIBM>
+__device__ __forceinline__ float tile_div(float v, float sum, float rsum) {
+  if constexpr (LIBM)
+    return v / sum;
+  else
+    return v * rsum;
+}
+
+// the fused tiles' waves, and the entries of a row that they hold in
+// registers (each wave kFusedChunks chunks of 16)
+constexpr int kFusedCols = 512;
+constexpr int kFusedWaves = 8;
+constexpr int kFusedChunks = kFusedCols / (16 * kFusedWaves);
+
+// The structure check of a tile whose last row holds more than kFusedCols
+// entries: row after row against the last row's columns, wave w rows w and
+// w + W (nt <= 16 = 2 W), 512 entries a trip as 16-byte windows.  A window
+// of a row before the last that holds a compared entry starts below bl <=
+// nnz - kFusedCols and is never moved; the last row's are read from
+// min(e, amax) and shifted.  Every thread of the workgroup calls it.
+template <int W>
+__device__ __forceinline__ bool long_tile_prefix_ok(
+    const int32_t *__restrict__ col, int32_t my_ro, int nt, int32_t bl,
+    int32_t len_last, uint32_t amax, int *verdict /* __shared__ int[W] */) {
+  const int wave = wave_in_group();
+  const int l = lane_id();
+  int32_t b[2], len[2];
+  bool ok = true;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int rr = wave + h * W;
+    const int rc = rr < nt - 1 ? rr : nt - 1; // the last row against itself
+    b[h] = __builtin_amdgcn_readlane(my_ro, rc);
+    len[h] = __builtin_amdgcn_readlane(my_ro, rc + 1) - b[h];
+    ok &= len[h] <= len_last;
+    if (rr >= nt - 1)
+      len[h] = 0; // nothing to compare
+  }
+  const int32_t most = std::min(std::max(len[0], len[1]), len_last);
+  for (int32_t t0 = 0; t0 < most; t0 += 8 * kWave) { // wave-uniform
+    v4i x[2][2], y[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int32_t t = t0 + 4 * (l + u * kWave);
+      auto at = [&](int32_t row) __attribute__((always_inline)) {
+        v4i z;
+        __builtin_memcpy(
+            &z, at_bytes(col, 4u * std::min((uint32_t)(row + t), amax)),
+            sizeof z);
+        return z;
+      };
+      y[u] = at(bl);
+      x[0][u] = at(b[0]);
+      x[1][u] = at(b[1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int32_t t = t0 + 4 * (l + u * kWave);
+      const uint32_t e = (uint32_t)(bl + t);
+      const uint32_t d = e - std::min(e, amax);
+      const v4i z = {d == 0 ? y[u].x : d == 1 ? y[u].y : d == 2 ? y[u].z
+                                                                : y[u].w,
+                     d == 0 ? y[u].y : d == 1 ? y[u].z : y[u].w,
+                     d == 0 ? y[u].z : y[u].w, y[u].w};
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          ok &= (t + m >= len[h]) | (x[h][u][m] == z[m]);
+    }
+  }
+  const bool mine = __builtin_amdgcn_ballot_w64(!ok) == 0;
+  if (l == 0)
+    verdict[wave] = mine;
+  __syncthreads();
+  ok = true;
+#pragma unroll
+  for (int w = 0; w < W; ++w)
+    ok &= verdict[w] != 0;
+  return ok;
+}
+
+// A 16-row tile with the shared column structure whose last row holds more
+// entries than the fused kernels keep in registers (kFusedCols): the same
+// chunks, products and roundings in three passes over the tile's chunks,
+// wave w taking the 16-entry chunks w, w + W, ...
+//   A. S^T = K_chunk Q^T; the scores, as their op stores them, go to the
+//      score buffer (each lane re-reads only what it wrote itself) and into
+//      the running row maxima;
+//   B. (after the maxima met in LDS) the exponentials' row sums;
+//   C. P = exp / sum, stored over the scores, and output = P V, 64 columns
+//      at a time, the waves' partial tiles summed through LDS.
+// The extra passes re-read 2 or 4 bytes per entry from L2, against a K^T
+// column and a V row per entry and 16 rows.  SO: pass A alone.  Every wave
+// of the workgroup calls it; returns with every output stored.
+// 16,384 positions of up to 768 entries, d = dv = 128, bf16: 2002 us row by
+// row, 80 us here; fp32 2039 and 126 us.  Without the K^T or the V gathers
+// it would take 71 or 68 us: two rounds of a chain of about twenty dependent
+// trips, two workgroups a CU.
+template <typename T, int KB, int W, bool IL, bool SO, bool NS, bool LIBM>
+__device__ __forceinline__ void attention_long_tile(
+    const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
+    const T *__restrict__ mask, const T *__restrict__ q,
+    const T *__restrict__ kt, const T *__restrict__ value, T *scores,
+    T *__restrict__ rmax, T *__restrict__ rsum, T *__restrict__ out,
+    int64_t cols, int32_t kdim, int64_t dv, float alpha, float beta,
+    uint32_t amax, int region, int r0, int nt, int32_t rbase, int32_t la,
+    int32_t bl, int32_t len_last,
+    const std::conditional_t<std::is_same_v<T, float>, float, v4u> (
+        &qb)[std::is_same_v<T, float> ? 16 * KB : 2 * KB],
+    float (&part)[W][4][4][kWave], float (&wred)[2][W][16],
+    int &v_nonfinite) {
+  constexpr bool kF32 = std::is_same_v<T, float>;
+  constexpr int S = kF32 ? 16 * KB : 2 * KB;
+  using Op = std::conditional_t<kF32, float, v4u>;
+  using Win = std::conditional_t<kF32, v4f, v2u>; // four entries
+  const int wave = wave_in_group();
+  const int l = lane_id(), i = l & 15, g = l >> 4;
+  // (its own copies of the strides: shared with the register path, their
+  // multiples stayed live through both and spilled)
+  asm volatile("" : "+s"(cols), "+s"(dv));
+  // the column of entry t0 + i of the last row (its final column past it)
+  auto column = [&](int32_t t0) __attribute__((always_inline)) {
+    return (uint32_t)*at_bytes(
+        col, 4u * (uint32_t)(bl + std::min(t0 + i, len_last - 1)));
+  };
+  // entries t0 + 4g .. + 3 of row i: a window read from min(e, amax)
+  auto window = [&](const T *p, int32_t t0) __attribute__((always_inline)) {
+    const uint32_t e = (uint32_t)(rbase + t0 + 4 * g);
+    const uint32_t w = std::min(e, amax);
+    Win y;
+    __builtin_memcpy(&y, at_bytes(p, (uint32_t)sizeof(T) * w), sizeof y);
+    return y;
+  };
+  auto entries = [&](const Win &y, int32_t t0, float (&x)[4])
+      __attribute__((always_inline)) {
+    const uint32_t e = (uint32_t)(rbase + t0 + 4 * g);
+    const uint32_t d = e - std::min(e, amax);
+    if constexpr (kF32) {
+      x[0] = d == 0 ? y.x : d == 1 ? y.y : d == 2 ? y.z : y.w;
+      x[1] = d == 0 ? y.y : d == 1 ? y.z : y.w;
+      x[2] = d == 0 ? y.z : y.w;
+      x[3] = y.w;
+    } else {
+      const uint64_t w = ((uint64_t)y.y << 32) | y.x;
+      const uint64_t z = d < 4 ? w >> (16 * d) : 0ull;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        x[v] = bf16_to_f32((uint16_t)(z >> (16 * v)));
+    }
+  };
+  auto valid = [&](int32_t t0, int v) __attribute__((always_inline)) {
+    return t0 + 4 * g + v < la;
+  };
+  auto store = [&](int32_t t0, const float (&x)[4])
+      __attribute__((always_inline)) {
+    T *dst = scores + rbase + t0 + 4 * g;
+    Win y;
+    if constexpr (kF32)
+      y = v4f{x[0], x[1], x[2], x[3]};
+    else
+      y = v2u{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+    if (valid(t0, 3)) {
+      __builtin_memcpy(dst, &y, sizeof y);
+    } else {
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+        if (valid(t0, v))
+          stv(dst + v, x[v]);
+    }
+  };
+  const uint32_t row_bytes = (uint32_t)sizeof(T) * (uint32_t)cols;
+  const __amdgpu_buffer_rsrc_t kt_rsrc =
+      buffer_rsrc(kt, (uint32_t)kdim * row_bytes);
+  auto gather_k = [&](uint32_t c, Op (&a)[S]) __attribute__((always_inline)) {
+    if constexpr (kF32) {
+      const uint32_t ko = 16u * g * row_bytes + 4u * c;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int st = 0; st < 16; ++st)
+          a[kb * 16 + st] = buffer_load_f32(kt_rsrc, ko,
+                                            (uint32_t)(kb * 64 + st) *
+                                                row_bytes);
+    } else {
+      const uint32_t ko = 2u * c + 8u * g * row_bytes;
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        a[s] = gather_kt8(kt + (int64_t)(32 * s) * cols, row_bytes, ko);
+    }
+  };
+  // A.  The next columns a step ahead (two chunks' gathers in flight
+  // measured no faster).
+  constexpr int CA = 1;
+  float m = -INFINITY;
+  uint32_t cn[CA];
+#pragma unroll
+  for (int h = 0; h < CA; ++h)
+    cn[h] = column(16 * (wave + W * h));
+  for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W * CA) {
+    Op a[CA][S];
+    Win mw[CA];
+#pragma unroll
+    for (int h = 0; h < CA; ++h) {
+      gather_k(cn[h], a[h]);
+      mw[h] = Win{};
+      if constexpr (!NS)
+        mw[h] = window(mask, t0 + 16 * W * h);
+    }
+#pragma unroll
+    for (int h = 0; h < CA; ++h)
+      cn[h] = column(t0 + 16 * W * (CA + h));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < CA; ++h) {
+      const int32_t th = t0 + 16 * W * h;
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (kF32) {
+        v4f acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < S; st += 2) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][st], qb[st], acc,
+                                                     0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              a[h][st + 1], qb[st + 1], acc1, 0, 0, 0);
+        }
+        acc += acc1;
+      } else {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          acc = mfma_16x16x32_bf16(a[h][s], qb[s], acc);
+      }
+      float x[4], sv[4];
+      entries(mw[h], th, x);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        sv[v] = as_stored<T>(combine_sddmm(
+            region, valid(th, v) ? x[v] : 0.0f, acc[v], alpha, beta));
+        if constexpr (!SO)
+          m = valid(th, v) ? maximumf(m, sv[v]) : m;
+      }
+      store(th, sv);
+    }
+  }
+  if constexpr (SO)
+    return;
+  m = maximumf(m, swizzle_xor16(m));
+  m = maximumf(m, shfl_xor32(m));
+  if (g == 0)
+    wred[0][wave][i] = m;
+  if (threadIdx.x == 0)
+    v_nonfinite = 0;
+  __syncthreads();
+  m = wred[0][0][i];
+#pragma unroll
+  for (int w = 1; w < W; ++w)
+    m = maximumf(m, wred[0][w][i]);
+  // B.
+  auto exps = [&](const Win &y, int32_t t0, float (&x)[4])
+      __attribute__((always_inline)) {
+    entries(y, t0, x);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float e = as_stored<T>(tile_exp<LIBM>(x[v] - m));
+      x[v] = valid(t0, v) ? e : 0.0f;
+    }
+  };
+  float sum = 0.0f;
+  for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 64 * W) {
+    Win y[4]; // chunks past the row hold nothing valid
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      y[h] = window(scores, t0 + 16 * W * h);
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float x[4];
+      exps(y[h], t0 + 16 * W * h, x);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        sum += x[v];
+    }
+  }
+  sum += swizzle_xor16(sum);
+  sum += shfl_xor32(sum);
+  if (g == 0)
+    wred[1][wave][i] = sum;
+  __syncthreads();
+  sum = wred[1][0][i];
+#pragma unroll
+  for (int w = 1; w < W; ++w)
+    sum += wred[1][w][i];
+  sum = as_stored<T>(sum);
+  const float rsum_i = 1.0f / sum;
+  if (wave == 0 && g == 0 && i < nt) {
+    stv(rmax + r0 + i, m);
+    stv(rsum + r0 + i, sum);
+  }
+  // C.  The next columns a step ahead; bf16 takes two 64-column blocks of
+  // the output in one pass over the entries.
+  constexpr int NB = kF32 ? 1 : 2, CC = 1;
+  bool nonfinite = false;
+  for (int64_t nb0 = 0; nb0 < dv; nb0 += 64 * NB) {
+    const int ntiles0 = (int)std::min<int64_t>(4, (dv - nb0) / 16);
+    const bool both = NB == 2 && nb0 + 64 < dv; // wave-uniform
+    v4f acc[NB][4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        acc[j][n] = v4f{0.f, 0.f, 0.f, 0.f};
+    uint32_t cc[CC];
+#pragma unroll
+    for (int h = 0; h < CC; ++h)
+      cc[h] = column(16 * (wave + W * h));
+    for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W * CC) {
+      Win y[CC], bq[CC][NB][4];
+#pragma unroll
+      for (int h = 0; h < CC; ++h) {
+        y[h] = window(scores, t0 + 16 * W * h);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const uint32_t cs = (uint32_t)__builtin_amdgcn_ds_bpermute(
+              (4 * g + st) << 2, (int)cc[h]);
+          if constexpr (IL || !kF32) {
+            const uint32_t vo = (uint32_t)sizeof(T) *
+                                (cs * (uint32_t)dv + 4u * (uint32_t)i);
+            bq[h][0][st] =
+                *reinterpret_cast<const Win *>(at_bytes(value + nb0, vo));
+            if constexpr (NB == 2) {
+              bq[h][1][st] = Win{};
+              if (both)
+                bq[h][1][st] = *reinterpret_cast<const Win *>(
+                    at_bytes(value + nb0 + 64, vo));
+            }
+          } else {
+            const uint32_t vo = 4u * (cs * (uint32_t)dv + (uint32_t)i);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+              const int nn = n < ntiles0 ? n : 0; // wave-uniform
+              bq[h][0][st][n] = *at_bytes(value + nb0 + 16 * nn, vo);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < CC; ++h)
+        cc[h] = column(t0 + 16 * W * (CC + h));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < CC; ++h) {
+        const int32_t th = t0 + 16 * W * h;
+        float p[4];
+        if (nb0 == 0) { // P from the scores, stored over them
+          exps(y[h], th, p);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            p[v] = as_stored<T>(tile_div<LIBM>(p[v], sum, rsum_i));
+            p[v] = valid(th, v) ? p[v] : 0.0f;
+          }
+          store(th, p);
+        } else { // P as the first pass stored it
+          entries(y[h], th, p);
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            p[v] = valid(th, v) ? p[v] : 0.0f;
+        }
+        if constexpr (kF32) {
+#pragma unroll
+          for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+              acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  p[st], bq[h][0][st][n], acc[0][n], 0, 0, 0);
+        } else {
+          const v2u pk = v2u{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+              const v2u bn = v2u{bf16_pair(bq[h][j][0], bq[h][j][1], n),
+                                 bf16_pair(bq[h][j][2], bq[h][j][3], n)};
+              acc[j][n] = mfma_16x16x16_bf16(pk, bn, acc[j][n]);
+            }
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+    const int64_t nb = nb0 + 64 * j;
+    if (nb >= dv)
+      break; // wave-uniform
+    const int ntiles = (int)std::min<int64_t>(4, (dv - nb) / 16);
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        part[wave][n][v][l] = acc[j][n][v];
+    __syncthreads();
+    if (wave < (IL || !kF32 ? 4 : ntiles)) {
+      // IL: wave w finishes rows 4g + w, columns nb + 4i .. nb + 4i + 3;
+      // else wave n the tile of columns nb + 16n + i, rows 4g + v
+      float o[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        o[x] = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+          o[x] += IL || !kF32 ? part[w][x][wave][l] : part[w][wave][x][l];
+      }
+      if constexpr (IL || !kF32) {
+        const int rr = 4 * g + wave;
+        if (rr < nt) {
+          T *dst = out + (int64_t)(r0 + rr) * dv + nb + 4 * i;
+          if constexpr (kF32)
+            *reinterpret_cast<v4f *>(dst) = v4f{o[0], o[1], o[2], o[3]};
+          else
+            *reinterpret_cast<v2u *>(dst) =
+                v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            nonfinite |= !__builtin_isfinite(o[x]);
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (4 * g + v < nt) {
+            stv(out + (int64_t)(r0 + 4 * g + v) * dv + nb + 16 * wave + i,
+                o[v]);
+            nonfinite |= !__builtin_isfinite(o[v]);
+          }
+      }
+      if (__builtin_amdgcn_ballot_w64(nonfinite) != 0 && l == 0)
+        v_nonfinite = 1;
+    }
+    __syncthreads();
+    }
+  }
+  // (the barrier above also made every wave's stored P visible)
+  if (v_nonfinite != 0) // workgroup-uniform
+    for (int r = r0 + wave; r < r0 + nt; r += W)
+      attention_row_output(ro, col, scores, value, out, r, dv);
+}
+
 // The attention chain fused over 16-row tiles (d = 64 * KB, dv % 16 == 0):
 // scores = alpha * Q K^T + beta * mask on the mask's positions, the row
 // softmax (rowMaximum, rowSum and the normalised scores written as the
@@ -623,10 +1090,6 @@ __device__ __forceinline__ void attention_row_softmax(
 // row from the stored scores, adding exactly each row's own entries.
 // Scheduling barriers keep each batch of loads together and in order, so
 // that waiting for one batch leaves the later ones in flight.
-constexpr int kFusedCols = 512;
-constexpr int kFusedWaves = 8;
-constexpr int kFusedChunks = kFusedCols / (16 * kFusedWaves);
-
 // The host guarantees that the byte offsets into mask / scores (positions),
 // K^T (kdim * cols) and V (cols * dv) fit 32 bits and that nnz >= 4
 // (amax = nnz - 4, the last 4-entry window of the mask).
@@ -648,7 +1111,14 @@ constexpr int kFusedChunks = kFusedCols / (16 * kFusedWaves);
 // words the lane loaded and without the softmax's two barriers.  Its time is
 // the floor of the tile's chain of memory trips.
 // (at most 128 VGPRs: the two workgroups of a CU need four waves per SIMD)
-template <int KB, int W, bool IL, bool SO, bool NS = false, bool FLOOR = false>
+// LIBM: see tile_exp (calls without mapping options).
+// LONG: tiles with the shared structure and rows past kFusedCols entries
+// take attention_long_tile instead of running row by row.  Its code beside
+// the register path makes the allocator spill there (configuration 5 19.2
+// -> 20.3 us, d = 128 31.0 -> 33.5 us; the bf16 kernel, which always has it,
+// 14.4 -> 14.6 us), so the host takes it for long rows only.
+template <int KB, int W, bool IL, bool SO, bool NS = false, bool FLOOR = false,
+          bool LIBM = false, bool LONG = false>
 __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused(
     const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
     const float *__restrict__ mask, const float *__restrict__ q,
@@ -711,6 +1181,16 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused(
     const uint32_t e = rbase + chunk_t0(k) + 4 * g;
     return e < amax ? e : amax;
   };
+  if constexpr (LONG) {
+    if (len_last > kFusedCols && // workgroup-uniform
+        long_tile_prefix_ok<W>(col, my_ro, nt, bl, len_last, amax, wshared)) {
+      attention_long_tile<float, KB, W, IL, SO, NS, LIBM>(
+          ro, col, mask, q, kt, value, scores, rmax, rsum, out, cols, kdim,
+          dv, alpha, beta, amax, region, r0, nt, rbase, la, bl, len_last, qa,
+          part, wred, v_nonfinite);
+      return;
+    }
+  }
   // The structure check and the LDS copy of the last row's column indices
   // share one batch of loads: wave w compares rows w and w + W (at most two,
   // nt <= 16 = 2W) against the last row, a row of at most kFusedCols entries
@@ -990,7 +1470,7 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused(
       if (chunk_t0(k) < len_last) { // wave-uniform
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float e = exp_by_exp2(sv[k][v] - m);
+          const float e = tile_exp<LIBM>(sv[k][v] - m);
           sv[k][v] = valid(k, v) ? e : 0.0f;
           sum += sv[k][v];
         }
@@ -1018,7 +1498,7 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused(
       }
 #pragma unroll
       for (int v = 0; v < 4; ++v) { // zero past the row: P V adds nothing
-        const float p = sv[k][v] * rsum_i;
+        const float p = tile_div<LIBM>(sv[k][v], sum, rsum_i);
         sv[k][v] = valid(k, v) ? p : 0.0f;
       }
       // entries t0(k) + 4g .. + 3 of row i: one (unaligned) vector store
@@ -1157,19 +1637,6 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused(
 //     gives a lane its values for all four tiles.
 // Every result is rounded to bf16 where the separate op would store it.
 
-// the eight K^T values K^T[32 s + 8 g + e][c] (e = 0..7) as four bf16 pairs;
-// base is K^T row 32 s, lane_off the byte offset of column c plus 8 g rows
-__device__ __forceinline__ v4u gather_kt8(const uint16_t *base,
-                                          uint32_t row_bytes,
-                                          uint32_t lane_off) {
-  uint32_t x[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    x[e] = *at_bytes(at_bytes(base, e * row_bytes), lane_off);
-  return v4u{x[0] | (x[1] << 16), x[2] | (x[3] << 16), x[4] | (x[5] << 16),
-             x[6] | (x[7] << 16)};
-}
-
 // SDDMM over 16-row tiles, bf16 (kdim = 64 * KB; the host guarantees that
 // 2 * kdim * cols and 2 * nnz fit 32 bits and that lhs is 16-byte aligned).
 template <int KB, int W>
@@ -1285,7 +1752,9 @@ __global__ __launch_bounds__(64 * W) void sddmm_tile_mfma_bf16(
 // (amax = nnz - 4) and that Q is 16-byte and V 8-byte aligned.
 // (at most 128 VGPRs: the two workgroups of a CU need four waves per SIMD)
 // FLOOR: the tile-floor diagnostic, as for the fp32 kernel above.
-template <int KB, int W, bool SO, bool NS = false, bool FLOOR = false>
+// LIBM: see tile_exp (calls without mapping options).
+template <int KB, int W, bool SO, bool NS = false, bool FLOOR = false,
+          bool LIBM = false>
 __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused_bf16(
     const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
     const uint16_t *__restrict__ mask, const uint16_t *__restrict__ q,
@@ -1347,6 +1816,16 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused_bf16(
     return e < amax ? e : amax;
   };
   uint64_t mw[kFusedChunks];
+  if constexpr (!FLOOR) {
+    if (len_last > kFusedCols && // workgroup-uniform
+        long_tile_prefix_ok<W>(col, my_ro, nt, bl, len_last, amax, wshared)) {
+      attention_long_tile<uint16_t, KB, W, true, SO, NS, LIBM>(
+          ro, col, mask, q, kt, value, scores, rmax, rsum, out, cols, kdim,
+          dv, alpha, beta, amax, region, r0, nt, rbase, la, bl, len_last, qb,
+          part, wred, v_nonfinite);
+      return;
+    }
+  }
   // The structure check and the products run together: each wave checks its
   // rows against the last row and computes its chunks with the last row's
   // columns right away; the verdict is read at the softmax's first barrier,
@@ -1596,7 +2075,7 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused_bf16(
       if (chunk_t0(k) < len_last) { // wave-uniform
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float e = as_stored<uint16_t>(exp_by_exp2(sv[k][v] - m));
+          const float e = as_stored<uint16_t>(tile_exp<LIBM>(sv[k][v] - m));
           sv[k][v] = valid(k, v) ? e : 0.0f;
           sum += sv[k][v];
         }
@@ -1622,7 +2101,7 @@ __global__ __launch_bounds__(64 * W, 4) void attention_tile_fused_bf16(
       float p[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        p[v] = valid(k, v) ? sv[k][v] * rsum_i : 0.0f;
+        p[v] = valid(k, v) ? tile_div<LIBM>(sv[k][v], sum, rsum_i) : 0.0f;
       pk[k] = v2u{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
       uint16_t *dst = scores + rbase + chunk_t0(k) + 4 * g;
       if (valid(k, 3)) {
@@ -1731,6 +2210,12 @@ int grid_for(int64_t work, int64_t per_block, const char *what,
 
 namespace sw {
 
+// Whether rows past kFusedCols entries are to be expected: more than 400
+// entries in the mean row.  Block masks whose rows hold up to 512 stay below
+// it (configuration 5: rows of up to 384, 345 in the mean), a causal mask of
+// 850 positions is past it.
+bool long_rows(int64_t rows, int64_t nnz) { return nnz / 400 > rows; }
+
 template <typename T>
 int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
                  const T *lhs, const T *rhs, T *out, int64_t rows,
@@ -1751,8 +2236,17 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
       if ((kdim == 64 || kdim == 128) && nnz >= 4 &&
           narrow_offsets(nnz, 1) && narrow_offsets(cols, kdim) &&
           (val == nullptr || out + nnz <= val || val + nnz <= out)) {
+        const bool lng = long_rows(rows, nnz);
 #define SW_SDDMM_FUSED(KB, NS)                                                \
-  hipLaunchKernelGGL((attention_tile_fused<KB, kFusedWaves, false, true, NS>),\
+  do {                                                                        \
+    if (lng)                                                                  \
+      SW_SDDMM_FUSED_AS(KB, NS, true);                                        \
+    else                                                                      \
+      SW_SDDMM_FUSED_AS(KB, NS, false);                                       \
+  } while (0)
+#define SW_SDDMM_FUSED_AS(KB, NS, LONG)                                       \
+  hipLaunchKernelGGL((attention_tile_fused<KB, kFusedWaves, false, true, NS,  \
+                                           false, false, LONG>),              \
                      sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st, ro, \
                      col, val, lhs, rhs, nullptr, out, nullptr, nullptr,      \
                      nullptr, (int32_t)rows, cols, (int32_t)kdim, (int64_t)0, \
@@ -1765,6 +2259,7 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
           SW_SDDMM_FUSED(2, false);
         else
           SW_SDDMM_FUSED(2, true);
+#undef SW_SDDMM_FUSED_AS
 #undef SW_SDDMM_FUSED
         return launch_check("SDDMM tile MFMA kernel");
       }
@@ -2029,6 +2524,30 @@ int rowwise_map_entry(const int32_t *row_offsets,
                                rows, map, o, as_stream(stream));
 }
 
+// No output range shares a byte with an input or with another output.
+struct Range {
+  const void *p;
+  int64_t bytes;
+};
+bool outputs_apart(std::initializer_list<Range> outs,
+                   std::initializer_list<Range> ins) {
+  auto apart = [](const Range &a, const Range &b) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a.p),
+                    y = reinterpret_cast<uintptr_t>(b.p);
+    return a.bytes <= 0 || b.bytes <= 0 || x + (uintptr_t)a.bytes <= y ||
+           y + (uintptr_t)b.bytes <= x;
+  };
+  for (const Range &o : outs) {
+    for (const Range &i : ins)
+      if (!apart(o, i))
+        return false;
+    for (const Range &p : outs)
+      if (&p != &o && !apart(o, p))
+        return false;
+  }
+  return true;
+}
+
 // The whole chain in one kernel per 16-row tile when the options ask for
 // matrix-core tiles and the shapes fit the fused kernel; returns true when it
 // was launched (rc holds the launch status).
@@ -2038,7 +2557,7 @@ bool launch_fused_attention(const int32_t *ro, const int32_t *col,
                             float *rmax, float *rsum, float *out,
                             int64_t rows, int64_t cols, int64_t nnz,
                             int64_t d, int64_t dv, float alpha, float beta,
-                            hipStream_t st, int *rc) {
+                            bool libm, hipStream_t st, int *rc) {
   if (!((d == 64 || d == 128) && dv > 0 && dv % 16 == 0 && nnz >= 4 &&
         narrow_offsets(nnz, 1) && narrow_offsets(cols, d) &&
         narrow_offsets(cols, dv)))
@@ -2049,12 +2568,26 @@ bool launch_fused_attention(const int32_t *ro, const int32_t *col,
     return true;
   // interleaved output tiles (configuration 5: 25.2 -> 24.0 us)
   const bool il = dv % 64 == 0 && aligned16(v) && aligned16(out);
+  const bool lng = long_rows(rows, nnz);
+#define SW_FUSED_AS(KB, IL, LIBM, LONG)                                       \
+  hipLaunchKernelGGL(                                                         \
+      (attention_tile_fused<KB, kFusedWaves, IL, false, false, false, LIBM,   \
+                            LONG>),                                           \
+      sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st,    \
+      ro, col, mask, q, kt, v, scores, rmax, rsum, out, (int32_t)rows, cols,  \
+      (int32_t)d, dv, alpha, beta, (uint32_t)(nnz - 4),                       \
+      (int)SW_SDDMM_AFFINE)
 #define SW_FUSED(KB, IL)                                                      \
-  hipLaunchKernelGGL((attention_tile_fused<KB, kFusedWaves, IL, false>),      \
-                     sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st, ro, \
-                     col, mask, q, kt, v, scores, rmax, rsum, out,            \
-                     (int32_t)rows, cols, (int32_t)d, dv, alpha, beta,        \
-                     (uint32_t)(nnz - 4), (int)SW_SDDMM_AFFINE)
+  do {                                                                        \
+    if (libm && lng)                                                          \
+      SW_FUSED_AS(KB, IL, true, true);                                        \
+    else if (libm)                                                            \
+      SW_FUSED_AS(KB, IL, true, false);                                       \
+    else if (lng)                                                             \
+      SW_FUSED_AS(KB, IL, false, true);                                       \
+    else                                                                      \
+      SW_FUSED_AS(KB, IL, false, false);                                      \
+  } while (0)
   if (d == 64 && il)
     SW_FUSED(1, true);
   else if (d == 64)
@@ -2064,6 +2597,7 @@ bool launch_fused_attention(const int32_t *ro, const int32_t *col,
   else
     SW_FUSED(2, false);
 #undef SW_FUSED
+#undef SW_FUSED_AS
   *rc = launch_check("fused attention kernel");
   return true;
 }
@@ -2074,7 +2608,7 @@ bool launch_fused_attention(const int32_t *ro, const int32_t *col,
                             uint16_t *scores, uint16_t *rmax, uint16_t *rsum,
                             uint16_t *out, int64_t rows, int64_t cols,
                             int64_t nnz, int64_t d, int64_t dv, float alpha,
-                            float beta, hipStream_t st, int *rc) {
+                            float beta, bool libm, hipStream_t st, int *rc) {
   if (!((d == 64 || d == 128) && dv > 0 && dv % 64 == 0 && nnz >= 4 &&
         aligned16(q) &&
         (reinterpret_cast<uintptr_t>(v) & 7u) == 0 &&
@@ -2086,17 +2620,26 @@ bool launch_fused_attention(const int32_t *ro, const int32_t *col,
   *rc = grid_for(rows, 16, "fused attention", &grid);
   if (*rc)
     return true;
+#define SW_FUSED_AS(KB, LIBM)                                                 \
+  hipLaunchKernelGGL(                                                         \
+      (attention_tile_fused_bf16<KB, kFusedWaves, false, false, false, LIBM>),\
+      sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st,    \
+      ro, col, mask, q, kt, v, scores, rmax, rsum, out, (int32_t)rows, cols,  \
+      (int32_t)d, dv, alpha, beta, (uint32_t)(nnz - 4),                       \
+      (int)SW_SDDMM_AFFINE)
 #define SW_FUSED(KB)                                                          \
-  hipLaunchKernelGGL((attention_tile_fused_bf16<KB, kFusedWaves, false>),     \
-                     sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st, ro, \
-                     col, mask, q, kt, v, scores, rmax, rsum, out,            \
-                     (int32_t)rows, cols, (int32_t)d, dv, alpha, beta,        \
-                     (uint32_t)(nnz - 4), (int)SW_SDDMM_AFFINE)
+  do {                                                                        \
+    if (libm)                                                                 \
+      SW_FUSED_AS(KB, true);                                                  \
+    else                                                                      \
+      SW_FUSED_AS(KB, false);                                                 \
+  } while (0)
   if (d == 64)
     SW_FUSED(1);
   else
     SW_FUSED(2);
 #undef SW_FUSED
+#undef SW_FUSED_AS
   *rc = launch_check("fused attention kernel");
   return true;
 }
@@ -2238,13 +2781,36 @@ int attention_entry(const int32_t *row_offsets, const int32_t *column_indices,
       (nnz > 0 && (!scores || !query || !transposed_key || (dv > 0 && !value))))
     return fail(SW_ERR_INVALID_ARGUMENT, "attention buffer pointer is null");
   hipStream_t st = as_stream(stream);
-  if (nnz > 0 && o.sddmm_lanes_per_row == 64 &&
-      streq(o.sddmm_mapping, "row-tile-mfma") &&
-      streq(o.spmm_mapping, "row-tile-mfma") &&
+  const bool fused = o.sddmm_lanes_per_row == 64 &&
+                     streq(o.sddmm_mapping, "row-tile-mfma") &&
+                     streq(o.spmm_mapping, "row-tile-mfma");
+  // A call that leaves every mapping and block size at its default asks for
+  // the chain and not for a schedule: it takes the one-kernel form too, with
+  // the separate ops' expf and division (LIBM), when no output buffer shares
+  // memory with another operand (the six kernels finish reading an operand
+  // before a later one writes).  3,001 positions of up to 384 entries,
+  // d = dv = 64, fp32: 536 us in six kernels, 12.4 us in one.
+  const bool defaults =
+      streq(o.sddmm_mapping, "thread-per-row") &&
+      streq(o.spmm_mapping, "thread-per-output") &&
+      o.sddmm_lanes_per_row == 1 && o.sddmm_block_size == 256 &&
+      o.row_reduction_block_size == 256 && o.rowwise_map_block_size == 256 &&
+      o.spmm_block_size == 256 &&
+      outputs_apart({{scores, nnz * (int64_t)sizeof(T)},
+                     {row_maximum, rows * (int64_t)sizeof(T)},
+                     {row_sum, rows * (int64_t)sizeof(T)},
+                     {output, rows * dv * (int64_t)sizeof(T)}},
+                    {{row_offsets, (rows + 1) * 4},
+                     {column_indices, nnz * 4},
+                     {mask_values, nnz * (int64_t)sizeof(T)},
+                     {query, rows * d * (int64_t)sizeof(T)},
+                     {transposed_key, d * cols * (int64_t)sizeof(T)},
+                     {value, cols * dv * (int64_t)sizeof(T)}});
+  if (nnz > 0 && (fused || defaults) &&
       launch_fused_attention(row_offsets, column_indices, mask_values, query,
                              transposed_key, value, scores, row_maximum,
                              row_sum, output, rows, cols, nnz, d, dv, alpha,
-                             beta, st, &rc))
+                             beta, !fused, st, &rc))
     return rc;
   if (nnz > 0) {
     rc = launch_sddmm<T>(row_offsets, column_indices, mask_values, query,

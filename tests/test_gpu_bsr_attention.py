@@ -413,8 +413,9 @@ FUSED = ("sddmm-mapping=row-tile-mfma sddmm-lanes-per-row=64 "
 
 def _long_prefix_csr():
     """Tiles with the shared (prefix) column structure whose last rows hold
-    700, 512 and 513 entries: the fused kernel keeps at most 512 scores per
-    row in LDS and computes longer tiles row by row."""
+    700, 512 and 513 entries: the fused fp32 kernel keeps at most 512 scores
+    per row in registers and, at this mean row length, computes longer tiles
+    row by row (the bf16 one in passes over them)."""
     rng = np.random.default_rng(41)
     cols = 900
     rows_cols = []
