@@ -267,7 +267,8 @@ int sw_bsr_slab_floor(const int32_t *block_row_offsets,
  * sparsewave.sddmm: output_values[p] = region(values[p], lhs[r,:] . rhs[:,c])
  * for every stored (r, c) at position p.  lhs[rows][kdim], rhs[kdim][cols]
  * row-major.  ThreadPerRowSDDMMPattern (SparseWaveToGPU.cpp:667-750).
- * sddmm-mapping=row-tile-mfma runs 16-row v_mfma_f32_16x16x4_f32 tiles for
+ * Rows of more than 96 entries in the mean (kdim 64 or 128) and
+ * sddmm-mapping=row-tile-mfma run 16-row v_mfma_f32_16x16x4_f32 tiles for
  * kdim in {64,128,256}; with kdim 64 or 128, at least 4 entries, and
  * output_values not overlapping values (or SW_SDDMM_DOT), the tiles are the
  * fused attention kernel's product phase.  Other kdim take one wave per row.
@@ -290,6 +291,35 @@ int sw_sddmm_csr_bf16(const int32_t *row_offsets,
                       uint16_t *output_values, int64_t rows, int64_t cols,
                       int64_t nnz, int64_t kdim, int combine, float alpha,
                       float beta, const sw_options *opts, void *stream);
+
+/*
+ * The same SDDMM with scratch memory from the caller.
+ * sw_sddmm_workspace_bytes (value_bytes 4 for fp32, 2 for bf16) says with how
+ * many bytes the call is faster, 0 where it has no use for any: given at
+ * least that many at a 16-byte aligned device address, rhs is transposed
+ * there first and each entry reads consecutive elements (graphs; block
+ * masks run on matrix-core tiles without it).  A null, short or misaligned
+ * workspace is ignored.  The workspace belongs to the call until its work
+ * on `stream` is done.
+ */
+int64_t sw_sddmm_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz,
+                                 int64_t kdim, int value_bytes,
+                                 const sw_options *opts);
+int sw_sddmm_csr_f32_ws(const int32_t *row_offsets,
+                        const int32_t *column_indices, const float *values,
+                        const float *lhs, const float *rhs,
+                        float *output_values, int64_t rows, int64_t cols,
+                        int64_t nnz, int64_t kdim, int combine, float alpha,
+                        float beta, const sw_options *opts, void *workspace,
+                        int64_t workspace_bytes, void *stream);
+int sw_sddmm_csr_bf16_ws(const int32_t *row_offsets,
+                         const int32_t *column_indices,
+                         const uint16_t *values, const uint16_t *lhs,
+                         const uint16_t *rhs, uint16_t *output_values,
+                         int64_t rows, int64_t cols, int64_t nnz,
+                         int64_t kdim, int combine, float alpha, float beta,
+                         const sw_options *opts, void *workspace,
+                         int64_t workspace_bytes, void *stream);
 
 /*
  * sparsewave.csr_row_reduce: output[r] = fold over row r's stored values.

@@ -38,7 +38,8 @@ EXPORTED_SYMBOLS = (
     "sw_spmm_csr_f32", "sw_spmm_csr_bf16", "sw_bsr_spmm_f32",
     "sw_bsr_spmm_bf16", "sw_bsr_spmm_bf16_f32out", "sw_bsr_slab_floor",
     "sw_sddmm_csr_f32",
-    "sw_sddmm_csr_bf16", "sw_csr_row_reduce_f32", "sw_csr_row_reduce_bf16",
+    "sw_sddmm_csr_bf16", "sw_sddmm_workspace_bytes", "sw_sddmm_csr_f32_ws",
+    "sw_sddmm_csr_bf16_ws", "sw_csr_row_reduce_f32", "sw_csr_row_reduce_bf16",
     "sw_csr_rowwise_map_f32", "sw_csr_rowwise_map_bf16",
     "sw_sparse_attention_f32", "sw_sparse_attention_bf16",
     "sw_csr_row_at_position", "sw_attention_tile_floor",
@@ -136,6 +137,12 @@ def load_library():
                                             I64, ctypes.c_int, F, F, OP, P]),
         "sw_sddmm_csr_bf16": (ctypes.c_int, [P, P, P, P, P, P, I64, I64, I64,
                                              I64, ctypes.c_int, F, F, OP, P]),
+        "sw_sddmm_workspace_bytes": (I64, [I64, I64, I64, I64, ctypes.c_int,
+                                           OP]),
+        "sw_sddmm_csr_f32_ws": (ctypes.c_int, [P] * 6 + [I64] * 4 + [
+            ctypes.c_int, F, F, OP, P, I64, P]),
+        "sw_sddmm_csr_bf16_ws": (ctypes.c_int, [P] * 6 + [I64] * 4 + [
+            ctypes.c_int, F, F, OP, P, I64, P]),
         "sw_csr_row_reduce_f32": (ctypes.c_int, [P, P, P, P, I64, I64, C, OP,
                                                  P]),
         "sw_csr_row_reduce_bf16": (ctypes.c_int, [P, P, P, P, I64, I64, C, OP,
@@ -273,10 +280,30 @@ def _value_dtype(t, name):
     return t.dtype
 
 
-def _fn(base, dtype):
+def _fn(base, dtype, suffix=""):
     import torch
     return getattr(load_library(),
-                   base + ("_bf16" if dtype == torch.bfloat16 else "_f32"))
+                   base + ("_bf16" if dtype == torch.bfloat16 else "_f32") +
+                   suffix)
+
+
+def _workspace(nbytes, like, stream):
+    """Scratch memory for one call on `stream`, from torch's allocator (which
+    gives it again only to later work on that stream), or None where there
+    is none to be had: under graph capture, on a stream that is not torch's,
+    or out of memory."""
+    import torch
+    if stream is not None:
+        if not isinstance(stream, torch.cuda.Stream):
+            return None
+        with torch.cuda.stream(stream):
+            return _workspace(nbytes, like, None)
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def spmv(row_offsets, column_indices, values, vector, output, options=None,
@@ -469,12 +496,22 @@ def sddmm(row_offsets, column_indices, values, lhs, rhs, output_values,
         _need(values.numel() == nnz,
               "values must hold one value per stored entry")
     vals = values if combine != SDDMM_DOT else output_values
-    _check(_fn("sw_sddmm_csr", dt)(
-        _dev(row_offsets, torch.int32, "row_offsets"),
-        _dev(column_indices, torch.int32, "column_indices"),
-        _dev(vals, dt, "values"), _dev(lhs, dt, "lhs"), _dev(rhs, dt, "rhs"),
-        _dev(output_values, dt, "output_values"), rows, rhs.shape[1], nnz,
-        lhs.shape[1], combine, alpha, beta, _opts(options), _stream(stream)))
+    if isinstance(options, str):
+        options = Options.parse(options)
+    args = (_dev(row_offsets, torch.int32, "row_offsets"),
+            _dev(column_indices, torch.int32, "column_indices"),
+            _dev(vals, dt, "values"), _dev(lhs, dt, "lhs"),
+            _dev(rhs, dt, "rhs"), _dev(output_values, dt, "output_values"),
+            rows, rhs.shape[1], nnz, lhs.shape[1], combine, alpha, beta,
+            _opts(options))
+    need = load_library().sw_sddmm_workspace_bytes(
+        *args[6:10], output_values.element_size(), args[-1])
+    workspace = _workspace(need, rhs, stream) if need > 0 else None
+    if workspace is None:
+        _check(_fn("sw_sddmm_csr", dt)(*args, _stream(stream)))
+    else:
+        _check(_fn("sw_sddmm_csr", dt, "_ws")(
+            *args, workspace.data_ptr(), need, _stream(stream)))
     return output_values
 
 

@@ -351,6 +351,142 @@ __global__ __launch_bounds__(64 * W) void sddmm_tile_mfma(
   }
 }
 
+// ---- SDDMM over a transposed rhs --------------------------------------------
+// A stored entry's dot product reads a column of rhs, kdim elements a row of
+// rhs apart: where neighbouring entries do not share the cache lines (a
+// graph's columns) every element is a line of its own.  With scratch memory
+// for the transposed rhs (the _ws entry points) it is transposed once, and
+// an entry reads kdim consecutive elements.
+
+// rhs[kdim][cols] as rhst[cols][kp], columns of kp >= kdim elements (a
+// multiple of 16 bytes), zero past kdim.  64 x 64 tiles through LDS, both
+// sides in whole lines.
+template <typename T>
+__global__ __launch_bounds__(256) void transpose_rhs(
+    const T *__restrict__ rhs, T *__restrict__ rhst, int64_t cols,
+    int32_t kdim, int32_t kp, int64_t col_tiles) {
+  __shared__ T tile[64][64 + 4 / sizeof(T)];
+  const int64_t id = block_id();
+  const int64_t kt = id / col_tiles;
+  const int64_t c0 = (id - kt * col_tiles) * 64;
+  const int32_t k0 = (int32_t)kt * 64;
+  if (k0 >= kp)
+    return; // a folded grid's surplus workgroup (workgroup-uniform)
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int32_t k = k0 + 4 * u + y;
+    tile[4 * u + y][x] =
+        k < kdim && c0 + x < cols ? rhs[(int64_t)k * cols + c0 + x] : T(0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int64_t c = c0 + 4 * u + y;
+    if (c < cols && k0 + x < kp)
+      rhst[c * kp + k0 + x] = tile[x][4 * u + y];
+  }
+}
+
+// A wave takes 64 consecutive positions, lane l holding position l's row
+// (wave-uniform searches for the first and last, then its own between them),
+// column and sample.  G lanes compute an entry's dot product, V = 16 bytes'
+// worth of elements a lane and step from the lhs row and the transposed
+// column, 64 / G entries at a time and U such steps' loads in flight; the
+// sums return to the entries' lanes, whose stores are consecutive.  The work
+// is cut by entries, so rows of any length cost the same.
+// It is bound by the gathered columns' trips from L2 and the MALL (246 MB).
+// 60,013 x 50,021, 960,000 entries, kdim = 64, fp32: 1904 us one thread per
+// row, 643 one wave per row, 48.7 here, 12.4 of them the transposition.
+template <typename T, int G>
+__global__ __launch_bounds__(256) void sddmm_positions(
+    const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
+    const T *val, const T *__restrict__ lhs, const T *__restrict__ rhst,
+    T *out, int32_t rows, int32_t nnz, int32_t kdim, int32_t kp, int kind,
+    float alpha, float beta) {
+  constexpr int V = 16 / (int)sizeof(T);
+  constexpr int E = kWave / G; // entries a step
+  constexpr int U = G < 4 ? G : 4;
+  using Vec = std::conditional_t<sizeof(T) == 4, v4f, v4u>;
+  const int64_t first =
+      (block_id() * (blockDim.x / kWave) + wave_in_group()) * kWave;
+  if (first >= nnz)
+    return; // wave-uniform
+  const int l = lane_id(), gl = l & (G - 1), q = l / G;
+  const int32_t n = (int32_t)std::min<int64_t>(kWave, nnz - first);
+  // (lanes past the end repeat the last position)
+  const int32_t p = (int32_t)first + std::min(l, n - 1);
+  const int32_t c = col[p];
+  const float sample = val != nullptr ? ldv(val + p) : 0.0f;
+  const int fr = row_search_uniform(ro, 1u, (uint32_t)rows + 1u,
+                                    (int32_t)first);
+  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows + 1u,
+                                   (int32_t)first + n - 1);
+  const int32_t r = row_search_lane(ro, (uint32_t)fr + 1u, (uint32_t)lr + 2u,
+                                    p);
+  float mine = 0.0f;
+  for (int e0 = 0; e0 < n; e0 += E * U) { // wave-uniform
+    float dot[U];
+    int32_t rr[U], cc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int src = (e0 + E * u + q) << 2; // < 64: E U divides 64
+      rr[u] = __builtin_amdgcn_ds_bpermute(src, r);
+      cc[u] = __builtin_amdgcn_ds_bpermute(src, c);
+      dot[u] = 0.0f;
+    }
+    for (int32_t k0 = 0; k0 < kdim; k0 += G * V) {
+      const int32_t k = k0 + gl * V;
+      Vec a[U], b[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        a[u] = b[u] = Vec{};
+      if (k < kdim) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          b[u] = *reinterpret_cast<const Vec *>(rhst + (int64_t)cc[u] * kp +
+                                                k);
+        // (a lhs row ends at kdim, the next one's elements must not be read
+        // past the last row's end)
+        if (k + V <= kdim) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            __builtin_memcpy(&a[u], lhs + (int64_t)rr[u] * kdim + k,
+                             sizeof(Vec));
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            T x[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+              x[v] = k + v < kdim ? lhs[(int64_t)rr[u] * kdim + k + v] : T(0);
+            __builtin_memcpy(&a[u], x, sizeof x);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        T x[V], y[V];
+        __builtin_memcpy(x, &a[u], sizeof x);
+        __builtin_memcpy(y, &b[u], sizeof y);
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          dot[u] = __builtin_fmaf(tof(x[v]), tof(y[v]), dot[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float sum = group_sum<G>(dot[u]);
+      // entry e0 + E u + j was computed by the lanes G j .. G j + G - 1
+      const float s = __int_as_float(__builtin_amdgcn_ds_bpermute(
+          (G * (l & (E - 1))) << 2, __float_as_int(sum)));
+      mine = l / E == (e0 / E) + u ? s : mine;
+    }
+  }
+  if (l < n)
+    stv(out + p, combine_sddmm(kind, sample, mine, alpha, beta));
+}
+
 template <bool MAX, typename T>
 __global__ __launch_bounds__(1024) void row_reduce_thread(
     const int32_t *__restrict__ ro, const T *__restrict__ val,
@@ -2216,15 +2352,106 @@ namespace sw {
 // 850 positions is past it.
 bool long_rows(int64_t rows, int64_t nnz) { return nnz / 400 > rows; }
 
+// Rows of more than 96 entries in the mean are taken for a block mask's,
+// which the 16-row matrix-core tiles share their columns on; those of a
+// graph are shorter.  (Tiles without shared columns run row by row, one wave
+// each: 4,096 rows of 100 random columns, kdim = 64, 46 us, one thread per
+// row 645.)
+bool block_rows(int64_t rows, int64_t nnz) { return nnz / 96 >= rows; }
+
+// The 16-row tiles of the fused attention kernel's product phase serve this
+// call: asked for, or rows long enough.  (kdim 256 and bf16's or fp32's other
+// tile kernels are chosen in launch_sddmm.)
+bool sddmm_tiles(int64_t rows, int64_t nnz, int64_t kdim,
+                 const sw_options &o) {
+  return streq(o.sddmm_mapping, "row-tile-mfma") ||
+         ((kdim == 64 || kdim == 128) && block_rows(rows, nnz));
+}
+
+// Below this many multiply-adds a call is bound by its launches: one wave per
+// row without preparation (1,000 rows of 10, kdim = 16: 9.2 us against 17 with
+// the transposition, 30 one thread per row; 2,000 rows of 32, kdim = 96,
+// 6.2 M: 15.2 / 17.6 / 85; 4,096 rows of 90, kdim = 64, 24 M: 50 / 17.7 /
+// 587).
+bool small_sddmm(int64_t nnz, int64_t kdim) { return nnz < 8000000 / kdim; }
+
+// Bytes of scratch memory with which launch_sddmm transposes rhs first (0:
+// it would not).  A transposition reads and writes rhs once, a gathered
+// column costs a line per element: worth it from one entry per four columns
+// on, and not for block masks, whose gathers share their lines (8,192 rows of
+// 345 entries, kdim = 96: 71 us one wave per row, 94 transposed).  At most
+// 1 GiB.
+int64_t sddmm_workspace(int64_t rows, int64_t cols, int64_t nnz, int64_t kdim,
+                        int64_t elem, const sw_options &o) {
+  if (rows <= 0 || cols <= 0 || kdim <= 0 || kdim > INT32_MAX / 2 ||
+      small_sddmm(nnz, kdim) || nnz < cols / 4 || block_rows(rows, nnz) ||
+      (streq(o.sddmm_mapping, "row-tile-mfma") &&
+       (kdim == 64 || kdim == 128 || kdim == 256)))
+    return 0;
+  const int64_t kp = ceil_div(kdim, 16 / elem) * (16 / elem);
+  if (cols > ((int64_t)1 << 30) / (kp * elem))
+    return 0;
+  return cols * kp * elem;
+}
+
+template <typename T>
+int launch_sddmm_transposed(const int32_t *ro, const int32_t *col,
+                            const T *val, const T *lhs, const T *rhs, T *out,
+                            int64_t rows, int64_t cols, int64_t nnz,
+                            int64_t kdim, int kind, float alpha, float beta,
+                            T *rhst, hipStream_t st) {
+  constexpr int64_t V = 16 / sizeof(T);
+  const int64_t kp = ceil_div(kdim, V) * V;
+  const int64_t col_tiles = ceil_div(cols, 64);
+  const int64_t tiles = col_tiles * ceil_div(kp, 64);
+  int rc = check_grid(tiles, 256, "SDDMM rhs transposition");
+  if (rc)
+    return rc;
+  hipLaunchKernelGGL(transpose_rhs<T>, grid_dim(tiles, 256), dim3(256), 0, st,
+                     rhs, rhst, cols, (int32_t)kdim, (int32_t)kp, col_tiles);
+  rc = launch_check("SDDMM rhs transposition kernel");
+  if (rc)
+    return rc;
+  const int64_t grid = ceil_div(nnz, 256);
+  rc = check_grid(grid, 256, "SDDMM");
+  if (rc)
+    return rc;
+  // lanes per entry: one 16-byte step of the dot product, at most 16 lanes
+  const int64_t steps = kp / V;
+#define SW_POS(G)                                                             \
+  hipLaunchKernelGGL((sddmm_positions<T, G>), grid_dim(grid, 256), dim3(256), \
+                     0, st, ro, col, val, lhs, rhst, out, (int32_t)rows,      \
+                     (int32_t)nnz, (int32_t)kdim, (int32_t)kp, kind, alpha,   \
+                     beta)
+  if (steps <= 2)
+    SW_POS(2);
+  else if (steps <= 4)
+    SW_POS(4);
+  else if (steps <= 8)
+    SW_POS(8);
+  else
+    SW_POS(16);
+#undef SW_POS
+  return launch_check("SDDMM kernel");
+}
+
+// (ws: at least sddmm_workspace bytes, 16-byte aligned, or null)
 template <typename T>
 int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
                  const T *lhs, const T *rhs, T *out, int64_t rows,
                  int64_t cols, int64_t nnz, int64_t kdim, int kind,
                  float alpha, float beta, const sw_options &o,
-                 hipStream_t st) {
+                 hipStream_t st, T *ws = nullptr) {
   int64_t grid;
-  if (streq(o.sddmm_mapping, "row-tile-mfma") &&
-      (kdim == 64 || kdim == 128 || kdim == 256)) {
+  if (ws != nullptr)
+    return launch_sddmm_transposed<T>(ro, col, val, lhs, rhs, out, rows, cols,
+                                      nnz, kdim, kind, alpha, beta, ws, st);
+  const bool apart = val == nullptr || out + nnz <= val || val + nnz <= out;
+  if (streq(o.sddmm_mapping, "row-tile-mfma")
+          ? kdim == 64 || kdim == 128 || kdim == 256
+          : sddmm_tiles(rows, nnz, kdim, o) && apart && nnz >= 4 &&
+                narrow_offsets(nnz, 1) && narrow_offsets(cols, kdim) &&
+                (sizeof(T) == 4 || aligned16(lhs))) {
     const int kb = (int)(kdim / 64);
     if constexpr (sizeof(T) == 4) {
       int rc = grid_for(rows, 16, "SDDMM", &grid);
@@ -2234,8 +2461,7 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
       // output apart from them: the fused attention kernel's product phase
       // (its 4-entry sample windows may reach a neighbouring tile's entries)
       if ((kdim == 64 || kdim == 128) && nnz >= 4 &&
-          narrow_offsets(nnz, 1) && narrow_offsets(cols, kdim) &&
-          (val == nullptr || out + nnz <= val || val + nnz <= out)) {
+          narrow_offsets(nnz, 1) && narrow_offsets(cols, kdim) && apart) {
         const bool lng = long_rows(rows, nnz);
 #define SW_SDDMM_FUSED(KB, NS)                                                \
   do {                                                                        \
@@ -2285,8 +2511,7 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
         return rc;
       // d of 64 or 128, and no sample values or an output apart from them:
       // the fused attention kernel's product phase, as for fp32
-      if ((kdim == 64 || kdim == 128) && nnz >= 4 &&
-          (val == nullptr || out + nnz <= val || val + nnz <= out)) {
+      if ((kdim == 64 || kdim == 128) && nnz >= 4 && apart) {
 #define SW_SDDMM_FUSED(KB, NS)                                                \
   hipLaunchKernelGGL((attention_tile_fused_bf16<KB, kFusedWaves, true, NS>),  \
                      sw::grid_dim(grid, 64 * kFusedWaves), dim3(64 * kFusedWaves), 0, st, ro, \
@@ -2319,9 +2544,13 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
       return launch_check("SDDMM tile MFMA kernel");
     }
   }
+  // (thread-per-row: only many short rows without scratch memory; rows of a
+  // block mask past its kernels' kdim, 8,192 of 345 entries, kdim = 96, take
+  // 562 us one thread per row, 71 one wave)
   if (streq(o.sddmm_mapping, "wave-per-row") ||
       (streq(o.sddmm_mapping, "row-tile-mfma")) ||
-      o.sddmm_lanes_per_row == 64) {
+      o.sddmm_lanes_per_row == 64 || small_sddmm(nnz, std::max<int64_t>(kdim, 1)) ||
+      block_rows(rows, nnz)) {
     int rc = grid_for(rows, 4, "SDDMM", &grid);
     if (rc)
       return rc;
@@ -2442,7 +2671,7 @@ int sddmm_entry(const int32_t *row_offsets, const int32_t *column_indices,
                 const T *values, const T *lhs, const T *rhs, T *output_values,
                 int64_t rows, int64_t cols, int64_t nnz, int64_t kdim,
                 int combine, float alpha, float beta, const sw_options *opts,
-                void *stream) {
+                void *workspace, int64_t workspace_bytes, void *stream) {
   clear_error();
   sw_options o;
   int rc = resolve_options(opts, &o);
@@ -2466,10 +2695,14 @@ int sddmm_entry(const int32_t *row_offsets, const int32_t *column_indices,
     return SW_OK;
   if (!output_values || (kdim > 0 && (!lhs || !rhs)))
     return fail(SW_ERR_INVALID_ARGUMENT, "SDDMM operand pointer is null");
+  const int64_t need =
+      workspace ? sddmm_workspace(rows, cols, nnz, kdim, sizeof(T), o) : 0;
+  const bool use = need > 0 && workspace_bytes >= need && aligned16(workspace);
   return launch_sddmm<T>(row_offsets, column_indices,
                          combine == SW_SDDMM_DOT ? nullptr : values, lhs, rhs,
                          output_values, rows, cols, nnz, kdim, combine, alpha,
-                         beta, o, as_stream(stream));
+                         beta, o, as_stream(stream),
+                         use ? static_cast<T *>(workspace) : nullptr);
 }
 
 template <typename T>
@@ -2873,7 +3106,44 @@ extern "C" int sw_sddmm_csr_f32(const int32_t *row_offsets,
                                 void *stream) {
   return sw::sddmm_entry<float>(row_offsets, column_indices, values, lhs, rhs,
                                 output_values, rows, cols, nnz, kdim, combine,
-                                alpha, beta, opts, stream);
+                                alpha, beta, opts, nullptr, 0, stream);
+}
+
+extern "C" int sw_sddmm_csr_f32_ws(
+    const int32_t *row_offsets, const int32_t *column_indices,
+    const float *values, const float *lhs, const float *rhs,
+    float *output_values, int64_t rows, int64_t cols, int64_t nnz,
+    int64_t kdim, int combine, float alpha, float beta, const sw_options *opts,
+    void *workspace, int64_t workspace_bytes, void *stream) {
+  return sw::sddmm_entry<float>(row_offsets, column_indices, values, lhs, rhs,
+                                output_values, rows, cols, nnz, kdim, combine,
+                                alpha, beta, opts, workspace, workspace_bytes,
+                                stream);
+}
+
+extern "C" int sw_sddmm_csr_bf16_ws(
+    const int32_t *row_offsets, const int32_t *column_indices,
+    const uint16_t *values, const uint16_t *lhs, const uint16_t *rhs,
+    uint16_t *output_values, int64_t rows, int64_t cols, int64_t nnz,
+    int64_t kdim, int combine, float alpha, float beta, const sw_options *opts,
+    void *workspace, int64_t workspace_bytes, void *stream) {
+  return sw::sddmm_entry<uint16_t>(
+      row_offsets, column_indices, values, lhs, rhs, output_values, rows, cols,
+      nnz, kdim, combine, alpha, beta, opts, workspace, workspace_bytes,
+      stream);
+}
+
+extern "C" int64_t sw_sddmm_workspace_bytes(int64_t rows, int64_t cols,
+                                            int64_t nnz, int64_t kdim,
+                                            int value_bytes,
+                                            const sw_options *opts) {
+  if (value_bytes != 4 && value_bytes != 2)
+    return 0;
+  if (opts)
+    return sw::sddmm_workspace(rows, cols, nnz, kdim, value_bytes, *opts);
+  sw_options o;
+  sw_options_init(&o);
+  return sw::sddmm_workspace(rows, cols, nnz, kdim, value_bytes, o);
 }
 
 extern "C" int sw_sddmm_csr_bf16(const int32_t *row_offsets,
@@ -2886,7 +3156,8 @@ extern "C" int sw_sddmm_csr_bf16(const int32_t *row_offsets,
                                  void *stream) {
   return sw::sddmm_entry<uint16_t>(row_offsets, column_indices, values, lhs,
                                    rhs, output_values, rows, cols, nnz, kdim,
-                                   combine, alpha, beta, opts, stream);
+                                   combine, alpha, beta, opts, nullptr, 0,
+                                   stream);
 }
 
 extern "C" int sw_csr_row_reduce_f32(const int32_t *row_offsets,

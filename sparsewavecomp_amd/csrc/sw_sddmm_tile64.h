@@ -154,7 +154,10 @@ __device__ __forceinline__ bool sddmm_tile64(
 #pragma unroll
       for (int j = 0; j < kCheckRows; ++j) {
         const int row = i0 + j < nt - 1 ? i0 + j : nt - 1;
-        const int32_t n = __builtin_amdgcn_readlane(rlen, row);
+        // (the last row, which repeats past the tile, is not compared: its
+        // final window may have moved)
+        const int32_t n =
+            row < nt - 1 ? __builtin_amdgcn_readlane(rlen, row) : 0;
         const int32_t lim = n < len_last ? n : len_last; // wave-uniform
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
