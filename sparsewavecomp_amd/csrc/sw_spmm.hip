@@ -13,89 +13,122 @@
 #include "sw_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace swd;
 
 namespace {
 
-// thread-per-output: one thread per C[r, c], sequential over the row.
-// Products are added in position order with kOutputDeep positions' loads
-// and rhs gathers in flight while that many remain, then four: the kernel's
-// time is the longest rows' chain of memory trips.
-constexpr int kOutputDeep = 16;
+// A row's outputs by a group of G lanes, for any k >= V and any alignment:
+// CL lanes of V consecutive columns each (a 16-byte load of an rhs row, or
+// what k allows, so that a gathered row is read by one instruction and once),
+// PL = G / CL entries at a time and U such steps in flight; the entry lanes'
+// sums meet in an xor butterfly.  A lane whose columns would pass k takes the
+// last V: it repeats some of its neighbour's and stores the same values.
+// Rows of more than kLongSteps steps are taken by the whole wave, one after
+// another (G < 64).  A row's sum has a fixed order.  Units run XCD-contiguous.
+// Bound by the gathered rows' trips from L2 and the MALL: 200,003 rows of 20
+// entries on average, k = 100, bf16: 268 us one thread per output, 187 us
+// here (0.8 GB of rhs rows).  The mapping thread-per-output: the reference's
+// one thread per output, whose wave waited for its longest row and loaded one
+// element a lane.
+constexpr int kRowSteps = 4;
+constexpr int kLongSteps = 8;
 
-// rhs[c][j].  NARROW (the host's guarantee that 4 * rhs_rows * k fits 32
-// bits): the wave-uniform base rhs plus a 32-bit lane byte offset, which the
-// load takes directly; otherwise a 64-bit lane address, whose multiply by k
-// costs more than the load (configuration 3, thread-per-output: K=64
-// 1797 -> 1381 us, K=4 685 -> 653 us with the narrow form).
-template <bool NARROW, typename T>
-__device__ __forceinline__ float rhs_at(const T *__restrict__ rhs, int32_t c,
-                                        int64_t k, int64_t j) {
-  if constexpr (NARROW)
-    return tof(*at_bytes(rhs, (uint32_t)sizeof(T) *
-                                  ((uint32_t)c * (uint32_t)k + (uint32_t)j)));
-  else
-    return ldv(rhs + (int64_t)c * k + j);
-}
-
-// ROW (k and the block size multiples of 64): a wave's 64 outputs lie in
-// one row, so the row index is put in a scalar register and the row's
-// column and value loads become scalar loads shared by the wave.
-template <bool NARROW, bool ROW, typename T>
-__global__ __launch_bounds__(1024) void spmm_thread_per_output(
+template <typename T, int V, int CL, int G>
+__global__ __launch_bounds__(256) void spmm_row_group(
     const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
     const T *__restrict__ val, const T *__restrict__ rhs,
-    T *__restrict__ out, int64_t rows, int64_t k) {
-  int64_t e = block_id() * blockDim.x + threadIdx.x;
-  if (e >= rows * k)
-    return;
-  int64_t r = e / k, c = e - r * k;
-  if constexpr (ROW) // rows * k < 2^31 * 64: the row fits 32 bits
-    r = __builtin_amdgcn_readfirstlane((int32_t)r);
-  int32_t s = ro[r], t = ro[r + 1];
-  float acc = 0.0f;
-  int32_t p = s;
-  for (; p + kOutputDeep - 1 < t; p += kOutputDeep) {
-    float v[kOutputDeep], b[kOutputDeep];
-    int32_t cc[kOutputDeep];
-#pragma unroll
-    for (int u = 0; u < kOutputDeep; ++u) {
-      v[u] = ldv(val + p + u);
-      cc[u] = col[p + u];
-    }
-#pragma unroll
-    for (int u = 0; u < kOutputDeep; ++u)
-      b[u] = rhs_at<NARROW>(rhs, cc[u], k, c);
-#pragma unroll
-    for (int u = 0; u < kOutputDeep; ++u)
-      acc = __builtin_fmaf(v[u], b[u], acc);
+    T *__restrict__ out, int64_t rows, int64_t k, int64_t tiles) {
+  constexpr int PL = G / CL, U = kRowSteps;
+  const int64_t unit =
+      xcd_contiguous(block_id(), grid_blocks()) * (256 / G) + threadIdx.x / G;
+  const int l = lane_id(), cl = l & (CL - 1);
+  int64_t r = unit, c0 = 0;
+  if (tiles > 1) {
+    r = unit / tiles;
+    c0 = (unit - r * tiles) * (CL * V);
   }
-  for (; p + 3 < t; p += 4) {
-    float v[4], b[4];
-    int32_t cc[4];
+  const bool in = r < rows;
+  const int32_t s = in ? ro[r] : 0, e = in ? ro[r + 1] : 0;
+  float acc[V];
+  // entries [b, end) of a row into acc, every PLn-th from b + first
+  auto add = [&](int32_t b, int32_t end, int64_t cb, bool live, int first,
+                 auto pln) __attribute__((always_inline)) {
+    constexpr int P = decltype(pln)::value;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      v[u] = ldv(val + p + u);
-      cc[u] = col[p + u];
+    for (int i = 0; i < V; ++i)
+      acc[i] = 0.0f;
+    if (!live)
+      return;
+    for (int32_t p = b + first; p < end; p += U * P) {
+      T x[U][V];
+      float v[U];
+      int64_t c[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int32_t q = std::min(p + u * P, end - 1);
+        v[u] = ldv(val + q);
+        c[u] = col[q];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        __builtin_memcpy(x[u], rhs + c[u] * k + cb, sizeof x[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const float y = __builtin_fmaf(v[u], tof(x[u][i]), acc[i]);
+          acc[i] = p + u * P < end ? y : acc[i];
+        }
     }
+  };
+  auto store = [&](int64_t row, int64_t cb) __attribute__((always_inline)) {
+    T o[V];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      b[u] = rhs_at<NARROW>(rhs, cc[u], k, c);
+    for (int i = 0; i < V; ++i)
+      stv(&o[i], acc[i]);
+    __builtin_memcpy(out + row * k + cb, o, sizeof o);
+  };
+  const bool wide = G < kWave && e - s > kLongSteps * U * PL;
+  const int gl = l & (G - 1);
+  const bool mine = in && c0 + cl * V < k;
+  const int64_t cb = std::min<int64_t>(c0 + cl * V, k - V);
+  add(s, e, cb, mine && !wide, gl / CL, std::integral_constant<int, PL>{});
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      acc = __builtin_fmaf(v[u], b[u], acc);
+  for (int off = CL; off < G; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      acc[i] += __shfl_xor(acc[i], off, 64);
+  if (mine && !wide && gl < CL)
+    store(r, cb);
+  if constexpr (G < kWave) {
+    uint64_t m = ballot(wide && gl == 0);
+    while (m != 0) { // wave-uniform
+      const int src = __builtin_ctzll(m);
+      m &= m - 1;
+      const int32_t ls = __builtin_amdgcn_readlane(s, src);
+      const int32_t le = __builtin_amdgcn_readlane(e, src);
+      const int64_t lc0 = __shfl(c0, src, 64), lr = __shfl(r, src, 64);
+      const int64_t lcb = std::min<int64_t>(lc0 + cl * V, k - V);
+      const bool ok = lc0 + cl * V < k;
+      add(ls, le, lcb, ok, l / CL, std::integral_constant<int, kWave / CL>{});
+#pragma unroll
+      for (int off = CL; off < kWave; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          acc[i] += __shfl_xor(acc[i], off, 64);
+      if (ok && l < CL)
+        store(lr, lcb);
+    }
   }
-  for (; p < t; ++p)
-    acc = __builtin_fmaf(ldv(val + p), rhs_at<NARROW>(rhs, col[p], k, c), acc);
-  stv(out + e, acc);
 }
 
 // wave-per-row-tile, Wave64 lane layout.
 //
 // wave-per-row-tile: one (row, tile) unit per group of G lanes, the units in
 // XCD-contiguous order (sw_spmm_tile.h holds the unit's code).
-template <int V, int CL, int G, typename T>
+template <int V, int CL, int G, typename T, bool ANY>
 __global__ __launch_bounds__(1024) void spmm_row_tile(
     const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
     const T *__restrict__ val, const T *__restrict__ rhs,
@@ -105,8 +138,9 @@ __global__ __launch_bounds__(1024) void spmm_row_tile(
   const int64_t unit =
       xcd_contiguous(block_id(), grid_blocks()) * units_per_block +
       threadIdx.x / G;
-  spmm_row_tile_unit<V, CL, G, T>(ro, col, val, rhs, out, rows, k, tile,
-                                  tiles_per_row, unit, threadIdx.x & (G - 1));
+  spmm_row_tile_unit<V, CL, G, T, ANY>(ro, col, val, rhs, out, rows, k, tile,
+                                       tiles_per_row, unit,
+                                       threadIdx.x & (G - 1));
 }
 
 __global__ __launch_bounds__(1024) void spmm_fill_zero(float *__restrict__ y,
@@ -818,16 +852,16 @@ __global__ __launch_bounds__(256) void spmm_row_owner(
   }
 }
 
-template <int V, int CL, int G, typename T>
+template <int V, int CL, int G, bool ANY, typename T>
 void launch_tile(int64_t grid, int64_t B, hipStream_t st, const int32_t *ro,
                  const int32_t *col, const T *val, const T *rhs, T *out,
                  int64_t rows, int64_t k, int32_t tile, int64_t tpr) {
-  hipLaunchKernelGGL((spmm_row_tile<V, CL, G, T>), sw::grid_dim(grid, B),
+  hipLaunchKernelGGL((spmm_row_tile<V, CL, G, T, ANY>), sw::grid_dim(grid, B),
                      dim3((unsigned)B), 0, st, ro, col, val, rhs, out, rows, k,
                      tile, tpr);
 }
 
-template <int V, int CL, typename T>
+template <int V, int CL, bool ANY, typename T>
 void dispatch_g(int G, int64_t rows, int64_t tpr, int64_t B, hipStream_t st,
                 const int32_t *ro, const int32_t *col, const T *val,
                 const T *rhs, T *out, int64_t k, int32_t tile,
@@ -840,9 +874,8 @@ void dispatch_g(int G, int64_t rows, int64_t tpr, int64_t B, hipStream_t st,
 #define SW_TILE_CASE(GG)                                                      \
   case GG:                                                                    \
     if constexpr (GG >= CL)                                                   \
-      launch_tile<V, CL, (GG >= CL ? GG : CL), T>(grid, B, st, ro, col, val,  \
-                                                  rhs, out, rows, k, tile,    \
-                                                  tpr);                       \
+      launch_tile<V, CL, (GG >= CL ? GG : CL), ANY, T>(                       \
+          grid, B, st, ro, col, val, rhs, out, rows, k, tile, tpr);           \
     break;
   switch (G) {
     SW_TILE_CASE(1)
@@ -872,6 +905,49 @@ int launch_position_init(const int32_t *ro, float *out, int64_t rows,
                          int64_t k, int64_t chunk, int64_t P, int64_t units,
                          int64_t waves, hipStream_t st);
 
+// spmm_row_group with its shape for these operands.
+template <typename T>
+int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
+                     const T *rhs, T *out, int64_t rows, int64_t nnz,
+                     int64_t k, const char *what, hipStream_t st) {
+  // V columns a lane: 16 bytes where k holds them.  CL lanes a row: past a
+  // mean of 48 entries more of them in flight are worth more than whole
+  // rows of rhs at once (fp32, 100,000 rows of 60, k = 128, CL 8 / 16 / 32:
+  // 464 / 531 / 618 us, k = 33 221 / 274; 200,003 rows of 20, k = 100 302 /
+  // 288 / 320).  PL entries at a time: 4 below a mean of 32 (k = 16, bf16,
+  // PL 4 / 16: rows of 20 43 / 50 us, of 60 57 / 52).
+  const int V = k >= 8 && sizeof(T) == 2 ? 8 : k >= 4 ? 4 : k >= 2 ? 2 : 1;
+  const int CL = next_pow2((int)std::min<int64_t>(
+      ceil_div(k, V), nnz / 48 >= rows ? 8 : 16));
+  const int G = std::min(64, CL * (nnz / 32 < rows ? 4 : 16));
+  const int64_t tiles = ceil_div(k, (int64_t)CL * V);
+  const int64_t grid =
+      std::max<int64_t>(ceil_div(rows * tiles, 256 / G), 1);
+  const int rc = check_grid(grid, 256, what);
+  if (rc)
+    return rc;
+  const dim3 g = grid_dim(grid, 256);
+#define SW_ROWS(VV, CC, GG)                                                   \
+  if (V == VV && CL == CC && G == GG)                                         \
+  hipLaunchKernelGGL((spmm_row_group<T, VV, CC, GG>), g, dim3(256), 0, st,  \
+                     ro, col, val, rhs, out, rows, k, tiles);
+#define SW_ROWS_V(VV)                                                         \
+  SW_ROWS(VV, 1, 4) SW_ROWS(VV, 1, 16) SW_ROWS(VV, 2, 8) SW_ROWS(VV, 2, 32)   \
+  SW_ROWS(VV, 4, 16) SW_ROWS(VV, 4, 64) SW_ROWS(VV, 8, 32)                    \
+  SW_ROWS(VV, 8, 64) SW_ROWS(VV, 16, 64)
+  if constexpr (sizeof(T) == 2) {
+    SW_ROWS_V(8)
+    SW_ROWS(4, 1, 4) SW_ROWS(4, 1, 16) SW_ROWS(4, 2, 8) SW_ROWS(4, 2, 32)
+  } else {
+    SW_ROWS_V(4)
+  }
+  SW_ROWS(2, 1, 4) SW_ROWS(2, 1, 16) SW_ROWS(2, 2, 8) SW_ROWS(2, 2, 32)
+  SW_ROWS(1, 1, 4) SW_ROWS(1, 1, 16)
+#undef SW_ROWS_V
+#undef SW_ROWS
+  return launch_check("SpMM row kernel");
+}
+
 // The mappings that need no partial sums in the output: thread-per-output,
 // row-tile-mfma, wave-per-row-balanced and wave-per-row-tile, for fp32 and
 // bf16.  Returns 1 (and sets *rc) when it handled the mapping.
@@ -886,25 +962,7 @@ bool launch_spmm_rows(const int32_t *ro, const int32_t *col, const T *val,
     return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0;
   };
   if (streq(o.spmm_mapping, "thread-per-output")) {
-    int64_t grid = std::max<int64_t>(ceil_div(rows * k, B), 1);
-    *rc = check_grid(grid, B, what);
-    if (*rc)
-      return true;
-    dim3 g = grid_dim(grid, B), b((unsigned)B);
-    const bool row = k % kWave == 0 && B % kWave == 0 && rows <= INT32_MAX;
-    if (narrow_offsets(rhs_rows, k) && row)
-      hipLaunchKernelGGL((spmm_thread_per_output<true, true, T>), g, b, 0, st,
-                         ro, col, val, rhs, out, rows, k);
-    else if (narrow_offsets(rhs_rows, k))
-      hipLaunchKernelGGL((spmm_thread_per_output<true, false, T>), g, b, 0,
-                         st, ro, col, val, rhs, out, rows, k);
-    else if (row)
-      hipLaunchKernelGGL((spmm_thread_per_output<false, true, T>), g, b, 0,
-                         st, ro, col, val, rhs, out, rows, k);
-    else
-      hipLaunchKernelGGL((spmm_thread_per_output<false, false, T>), g, b, 0,
-                         st, ro, col, val, rhs, out, rows, k);
-    *rc = launch_check("thread-per-output SpMM kernel");
+    *rc = launch_row_group<T>(ro, col, val, rhs, out, rows, nnz, k, what, st);
     return true;
   }
   if (streq(o.spmm_mapping, "row-tile-mfma")) {
@@ -985,39 +1043,53 @@ bool launch_spmm_rows(const int32_t *ro, const int32_t *col, const T *val,
                         streq(o.spmm_mapping, "wave-per-row-tile-lds");
   if (!row_tile && sizeof(T) == 4)
     return false; // fp32: the position schedule
-  // wave-per-row-tile (bf16 also for the shapes the mappings above decline)
-  const int T_ = (int)o.spmm_tile_size;
-  const int64_t tpr = ceil_div(k, T_);
-  const bool vec = (T_ % 4 == 0) && (k % 4 == 0) && vec_ok(rhs) && vec_ok(out);
-  const int V = vec ? 4 : 1;
-  const int CL = next_pow2(ceil_div(T_, V));
-  const int G = std::max<int>((int)o.spmm_lanes_per_row, CL);
-  int64_t grid = 0;
-  const int32_t tile = (int32_t)T_;
-#define SW_CL_CASE(VV, CC)                                                    \
-  if (V == VV && CL == CC)                                                    \
-    dispatch_g<VV, CC, T>(G, rows, tpr, B, st, ro, col, val, rhs, out, k,     \
-                          tile, &grid);
-  SW_CL_CASE(4, 1)
-  SW_CL_CASE(4, 2)
-  SW_CL_CASE(4, 4)
-  SW_CL_CASE(4, 8)
-  SW_CL_CASE(1, 1)
-  SW_CL_CASE(1, 2)
-  SW_CL_CASE(1, 4)
-  SW_CL_CASE(1, 8)
-  SW_CL_CASE(1, 16)
-  SW_CL_CASE(1, 32)
-#undef SW_CL_CASE
-  if (grid == 0) {
-    *rc = fail(SW_ERR_INVALID_OPTION,
-               "no wave-per-row-tile kernel for tile size %d", T_);
+  // wave-per-row-tile (bf16 also for the shapes the mappings above decline).
+  // bf16 and tiles wider than k leave half the row tile's bytes or lanes
+  // unused: spmm_row_group (200,003 rows of 20, tile 32, us: fp32 k = 2 193 /
+  // 28, k = 16 80 / 62; bf16 k = 33 147 / 98, k = 100 280 / 187).
+  if (sizeof(T) == 2 || k < o.spmm_tile_size) {
+    *rc = launch_row_group<T>(ro, col, val, rhs, out, rows, nnz, k, what, st);
     return true;
   }
-  *rc = check_grid(grid, B, what);
-  if (*rc)
-    return true;
-  *rc = launch_check("wave-per-row-tile SpMM kernel");
+  if constexpr (sizeof(T) == 4) {
+    const int T_ = (int)o.spmm_tile_size;
+    const int64_t tpr = ceil_div(k, T_);
+    const bool vec = (T_ % 4 == 0) && (k % 4 == 0) && vec_ok(rhs) && vec_ok(out);
+    const bool any = !vec && T_ % 4 == 0 && k >= 4;
+    const int V = vec || any ? 4 : 1;
+    const int CL = next_pow2(ceil_div(T_, V));
+    const int G = std::max<int>((int)o.spmm_lanes_per_row, CL);
+    int64_t grid = 0;
+    const int32_t tile = (int32_t)T_;
+#define SW_CL_CASE(VV, CC, ANY)                                               \
+    if (V == VV && CL == CC && any == ANY)                                      \
+      dispatch_g<VV, CC, ANY, T>(G, rows, tpr, B, st, ro, col, val, rhs, out,   \
+                                 k, tile, &grid);
+    SW_CL_CASE(4, 1, false)
+    SW_CL_CASE(4, 2, false)
+    SW_CL_CASE(4, 4, false)
+    SW_CL_CASE(4, 8, false)
+    SW_CL_CASE(4, 1, true)
+    SW_CL_CASE(4, 2, true)
+    SW_CL_CASE(4, 4, true)
+    SW_CL_CASE(4, 8, true)
+    SW_CL_CASE(1, 1, false)
+    SW_CL_CASE(1, 2, false)
+    SW_CL_CASE(1, 4, false)
+    SW_CL_CASE(1, 8, false)
+    SW_CL_CASE(1, 16, false)
+    SW_CL_CASE(1, 32, false)
+#undef SW_CL_CASE
+    if (grid == 0) {
+      *rc = fail(SW_ERR_INVALID_OPTION,
+                 "no wave-per-row-tile kernel for tile size %d", T_);
+      return true;
+    }
+    *rc = check_grid(grid, B, what);
+    if (*rc)
+      return true;
+    *rc = launch_check("wave-per-row-tile SpMM kernel");
+  }
   return true;
 }
 

@@ -24,7 +24,12 @@ constexpr int kTileUnroll = 4;
 
 // One group's (row, tile) unit `unit`; gl is the lane's index in its group.
 // Every lane of the wave must call it (the reduction crosses the group).
-template <int V, int CL, int G, typename T>
+// ANY (V = 4, k >= 4): k, rhs and out of any alignment.  The accesses are
+// element-aligned, and a lane whose four columns would pass k takes the last
+// four instead: it repeats columns of its neighbour, in the same order, and
+// stores the same values (k = 33, tile 32, fp32, 100,000 rows of 60: 948 us
+// one column and one position a lane, 230 us so).
+template <int V, int CL, int G, typename T, bool ANY = false>
 __device__ __forceinline__ void spmm_row_tile_unit(
     const int32_t *__restrict__ ro, const int32_t *__restrict__ col,
     const T *__restrict__ val, const T *__restrict__ rhs,
@@ -39,15 +44,24 @@ __device__ __forceinline__ void spmm_row_tile_unit(
     r = unit / tiles_per_row;
     c0 = (unit - r * tiles_per_row) * tile;
   }
-  const int64_t cb = c0 + (int64_t)cl * V;
+  int64_t cb = c0 + (int64_t)cl * V;
   const int64_t cend = std::min<int64_t>(c0 + tile, k);
+  const bool live = unit_ok && cb < cend;
+  if constexpr (ANY)
+    cb = std::min<int64_t>(cb, k - 4);
+  auto load4 = [](const T *p) __attribute__((always_inline)) {
+    if constexpr (ANY)
+      return ld4_any(p);
+    else
+      return ld4(p);
+  };
   float acc[V];
 #pragma unroll
   for (int i = 0; i < V; ++i)
     acc[i] = 0.0f;
-  if (unit_ok && cb < cend) {
+  if (live) {
     const int32_t s = ro[r], e = ro[r + 1];
-    if (V == 4 && cb + 4 <= cend) {
+    if (ANY || (V == 4 && cb + 4 <= cend)) {
       int32_t p = s + pl;
       // kTileUnroll positions per lane in flight: their loads and rhs
       // gathers are issued before the first product (rows longer than the
@@ -63,7 +77,7 @@ __device__ __forceinline__ void spmm_row_tile_unit(
         v4f b[kTileUnroll];
 #pragma unroll
         for (int u = 0; u < kTileUnroll; ++u)
-          b[u] = ld4(rhs + c[u] * k + cb);
+          b[u] = load4(rhs + c[u] * k + cb);
 #pragma unroll
         for (int u = 0; u < kTileUnroll; ++u) {
           acc[0] = __builtin_fmaf(v[u], b[u].x, acc[0]);
@@ -77,7 +91,7 @@ __device__ __forceinline__ void spmm_row_tile_unit(
       for (; p < e; p += PL) {
         const float v = tof(ld_stream(val + p));
         const int64_t c = ld_stream(col + p);
-        const v4f b = ld4(rhs + c * k + cb);
+        const v4f b = load4(rhs + c * k + cb);
         acc[0] = __builtin_fmaf(v, b.x, acc[0]);
         if constexpr (V == 4) {
           acc[1] = __builtin_fmaf(v, b.y, acc[1]);
@@ -104,8 +118,13 @@ __device__ __forceinline__ void spmm_row_tile_unit(
     for (int i = 0; i < V; ++i)
       acc[i] += __shfl_xor(acc[i], off, 64);
   }
-  if (unit_ok && pl == 0 && cb < cend) {
+  if (live && pl == 0) {
     T *o = out + r * k + cb;
+    if constexpr (ANY) {
+      st4_any(o, v4f{acc[0], acc[V > 1 ? 1 : 0], acc[V > 2 ? 2 : 0],
+                     acc[V > 3 ? 3 : 0]});
+      return;
+    }
     // non-temporal: the output is not re-read and should not displace RHS
     // rows from L2
     if (V == 4 && cb + 4 <= cend) {
