@@ -86,6 +86,18 @@ class _COptions(ctypes.Structure):
 
 
 _lib = None
+_torch = None
+
+
+def _load_torch():
+    """torch, imported when the first operand arrives and read from the module
+    afterwards: import statements and c_void_p objects on every call took 0.8
+    of the 6.9 us of a small SpMV (4,096 rows, 65,536 entries), of which the
+    C call is 3.9."""
+    global _torch
+    import torch
+    _torch = torch
+    return torch
 
 
 def library_path() -> str:
@@ -229,7 +241,7 @@ def _opts(options):
 
 
 def _dev(t, dtype, name):
-    import torch
+    torch = _torch or _load_torch()
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if not t.is_cuda:  # cheaper than building t.device on every call
@@ -238,19 +250,19 @@ def _dev(t, dtype, name):
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _stream(stream):
-    import torch
+    torch = _torch or _load_torch()
     if stream is None:
         # the current stream's handle without building a Stream object
         # (about 0.1 us against 2.8 us per call on the MI355X host)
         raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if raw is not None:
-            return ctypes.c_void_p(raw(torch.cuda.current_device()))
+            return raw(torch.cuda.current_device())
         stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return stream.cuda_stream
 
 
 class ShapeError(SparseWaveError, ValueError):
@@ -267,21 +279,22 @@ def _need(cond, message):
 
 
 def _rows_of(row_offsets, name="row_offsets"):
-    _need(row_offsets.dim() == 1 and row_offsets.numel() >= 1,
-          f"{name} must be a 1-D tensor of rows + 1 offsets")
-    return row_offsets.numel() - 1
+    n = row_offsets.numel()
+    if row_offsets.dim() != 1 or n < 1:  # no message built on good calls
+        raise ShapeError(f"{name} must be a 1-D tensor of rows + 1 offsets")
+    return n - 1
 
 
 def _value_dtype(t, name):
     """fp32 or bf16: the element type shared by an op's value operands."""
-    import torch
+    torch = _torch or _load_torch()
     if t.dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"{name} must be float32 or bfloat16, got {t.dtype}")
     return t.dtype
 
 
 def _fn(base, dtype, suffix=""):
-    import torch
+    torch = _torch or _load_torch()
     return getattr(load_library(),
                    base + ("_bf16" if dtype == torch.bfloat16 else "_f32") +
                    suffix)
@@ -292,7 +305,7 @@ def _workspace(nbytes, like, stream):
     gives it again only to later work on that stream), or None where there
     is none to be had: under graph capture, on a stream that is not torch's,
     or out of memory."""
-    import torch
+    torch = _torch or _load_torch()
     if stream is not None:
         if not isinstance(stream, torch.cuda.Stream):
             return None
@@ -309,13 +322,13 @@ def _workspace(nbytes, like, stream):
 def spmv(row_offsets, column_indices, values, vector, output, options=None,
          stream=None):
     """sparsewave.spmv (SparseWaveOps.td:17-52): output = A @ vector."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     _need(column_indices.numel() == values.numel(),
           "column indices and values must have the same length")
     _need(vector.dim() == 1, "vector must be 1-D")
-    _need(output.dim() == 1 and output.numel() == rows,
-          f"output must hold rows = {rows} values")
+    if output.dim() != 1 or output.numel() != rows:
+        raise ShapeError(f"output must hold rows = {rows} values")
     _check(load_library().sw_spmv_csr_f32(
         _dev(row_offsets, torch.int32, "row_offsets"),
         _dev(column_indices, torch.int32, "column_indices"),
@@ -330,7 +343,7 @@ def coo_spmv(row_indices, column_indices, values, vector, output,
              options=None, stream=None):
     """sparsewave.coo_spmv (SparseWaveOps.td:54-88): output = A @ vector with
     A as COO entries (any order, repeated coordinates add up)."""
-    import torch
+    torch = _torch or _load_torch()
     _need(row_indices.numel() == column_indices.numel() == values.numel(),
           "COO row indices, column indices and values must have the same "
           "length")
@@ -350,7 +363,7 @@ def spmv_gather_floor(column_indices, values, vector, partial, stream=None):
     """Diagnostic (no reference counterpart): partial[w] = sum of
     values[p] * vector[column_indices[p]] over p in [512 w, 512 w + 512),
     i.e. a CSR SpMV's column/value reads and x gathers without its rows."""
-    import torch
+    torch = _torch or _load_torch()
     nnz = values.numel()
     _need(column_indices.numel() == nnz,
           "column indices and values must have the same length")
@@ -368,7 +381,7 @@ def spmm(row_offsets, column_indices, values, rhs, output, options=None,
          stream=None):
     """sparsewave.spmm (SparseWaveOps.td:91-124): output = A @ rhs.  values,
     rhs and output share one element type, float32 or bfloat16."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     dt = _value_dtype(values, "values")
     _need(column_indices.numel() == values.numel(),
@@ -390,7 +403,7 @@ def bsr_spmm(block_row_offsets, block_column_indices, block_values, rhs,
     """sparsewave.bsr_spmm (SparseWaveOps.td:126-169).  float32 operands, or
     bfloat16 block values and rhs with a bfloat16 output (the op's
     same-element-type rule) or, as an extension, a float32 output."""
-    import torch
+    torch = _torch or _load_torch()
     _need(block_size >= 1, "block size must be positive")
     rows = _rows_of(block_row_offsets, "block_row_offsets") * block_size
     nnzb = block_column_indices.numel()
@@ -423,7 +436,7 @@ def bsr_slab_floor(block_row_offsets, block_column_indices, block_values,
     words each lane loads (sw_bsr_slab_floor); the output holds those XORs
     as bit patterns.  float32 operands, or bfloat16 block values and rhs with
     a bfloat16 or float32 output."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(block_row_offsets, "block_row_offsets") * 16
     nnzb = block_column_indices.numel()
     dt = _value_dtype(block_values, "block_values")
@@ -454,7 +467,7 @@ def attention_tile_floor(row_offsets, column_indices, mask_values, query,
     output reduction as they are and every product, exponential and
     division replaced by an XOR of the loaded words
     (sw_attention_tile_floor).  float32 or bfloat16 buffers."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     nnz = column_indices.numel()
     dt = _value_dtype(query, "query")
@@ -483,7 +496,7 @@ def attention_tile_floor(row_offsets, column_indices, mask_values, query,
 def sddmm(row_offsets, column_indices, values, lhs, rhs, output_values,
           combine=SDDMM_MUL, alpha=1.0, beta=0.0, options=None, stream=None):
     """sparsewave.sddmm (SparseWaveOps.td:171-223); float32 or bfloat16."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     nnz = column_indices.numel()
     dt = _value_dtype(output_values, "output_values")
@@ -518,7 +531,7 @@ def sddmm(row_offsets, column_indices, values, lhs, rhs, output_values,
 def csr_row_reduce(row_offsets, column_indices, values, output, kind="sum",
                    options=None, stream=None):
     """sparsewave.csr_row_reduce (SparseWaveOps.td:225-257)."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     dt = _value_dtype(values, "values")
     _need(output.numel() == rows, f"output must hold rows = {rows} values")
@@ -538,7 +551,7 @@ def csr_rowwise_map(row_offsets, column_indices, values, row_values,
                     output_values, kind=MAP_EXP_SUB, options=None,
                     stream=None):
     """sparsewave.csr_rowwise_map (SparseWaveOps.td:259-299)."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     dt = _value_dtype(values, "values")
     _need(row_values.numel() == rows,
@@ -564,7 +577,7 @@ def sparse_attention(row_offsets, column_indices, mask_values, query,
     """The six-op sparse attention chain
     (SparseAttentionToSparseWave.cpp:230-315), ten-buffer ABI; all value
     buffers float32, or all bfloat16 (the bf16 option)."""
-    import torch
+    torch = _torch or _load_torch()
     rows = _rows_of(row_offsets)
     nnz = column_indices.numel()
     dt = _value_dtype(query, "query")
@@ -595,7 +608,7 @@ def sparse_attention(row_offsets, column_indices, mask_values, query,
 
 def csr_row_at_position(row_offsets, positions, out_rows, stream=None):
     """sparsewave.csr_row_at_position for a batch (SparsePositionToSCF.cpp:225-271)."""
-    import torch
+    torch = _torch or _load_torch()
     _check(load_library().sw_csr_row_at_position(
         _dev(row_offsets, torch.int32, "row_offsets"),
         row_offsets.numel() - 1, _dev(positions, torch.int64, "positions"),
