@@ -579,7 +579,7 @@ def main():
             ms = time_steps(lambda: sw.coo_spmv(ri, col, val, xv, y,
                                                 options=o), K, Wm)
             workloads.setdefault("coo_spmv_config2", {})[
-                opts or "reference (thread-per-nonzero)"] = {
+                opts or "reference defaults"] = {
                 "ms": ms, "GB/s": coo_bytes / ms / 1e6,
                 "hbm_frac": coo_bytes / ms / 1e6 / HBM_PEAK_GBS}
             log(f"  {ms * 1e3:.1f} us  {coo_bytes / ms / 1e6:.0f} GB/s")
@@ -662,8 +662,7 @@ def main():
         workloads["spmv_config1"] = res1
 
         # ---- configuration 3: CSR SpMM K = 4 and 64 -------------------------
-        # the reference's default mapping (thread-per-output, 256-thread
-        # blocks) first, then this build's Wave64 mappings
+        # the default mapping first, then the others
         for k, opts in [(4, ""), (64, ""),
                         (4, "spmm-mapping=wave-per-position "
                             "spmm-positions-per-lane=8 spmm-block-size=256"),

@@ -5,7 +5,8 @@
  * (hipMalloc / torch CUDA tensor memory) unless stated otherwise; the caller
  * owns every buffer, outputs included.  All work is enqueued on `stream`
  * (a hipStream_t passed as void*, NULL = the default stream) with no host
- * synchronisation and no allocation.  Functions return SW_OK (0) or a
+ * synchronisation and no allocation; scratch memory, where an entry point can
+ * use it, is an argument.  Functions return SW_OK (0) or a
  * negative SW_ERR_* code; sw_last_error() then returns a message that
  * paraphrases the reference's diagnostic.  Index arrays are i32, values f32
  * (bf16 where the name says so).
@@ -25,8 +26,8 @@
  * (larger: SW_ERR_INVALID_SHAPE before any launch); COO takes any nnz.
  * Every mapping runs at those limits: a launch of more than 2^32 - 1
  * work-items, which one grid dimension cannot hold, is folded into a 2-D
- * grid, and a BSR SpMM whose block rows one grid dimension cannot hold
- * (past about 8.4 million) computes with its thread-per-output kernel.
+ * grid, and a BSR SpMM that the matrix-core kernels' grid cannot hold
+ * computes with its thread-per-output kernel.
  *
  * Citations are path:line into the reference (sott0n/SparseWaveComp).
  */
@@ -66,7 +67,9 @@ typedef struct sw_options {
   int64_t spmv_position_chunk_size; /* thread-per-position chunk, default 1 */
   char spmv_position_reduction[16]; /* atomic | segmented (thread-per-position) */
   int64_t position_block_size;      /* position-parallel init kernels, default 256 */
-  char spmm_mapping[32];            /* thread-per-output | wave-per-row-tile |
+  char spmm_mapping[32];            /* thread-per-output (lane groups over
+                                       whole rows of the rhs) |
+                                       wave-per-row-tile |
                                        thread-per-position | wave-per-position |
                                        row-tile-mfma | wave-per-row-balanced |
                                        wave-per-row-tile-lds (the last four
@@ -76,8 +79,9 @@ typedef struct sw_options {
   int64_t spmm_tile_size;           /* 1..32, default 4 */
   int64_t spmm_position_chunk_size; /* default 1 */
   int64_t sddmm_block_size;         /* default 256 */
-  int64_t row_reduction_block_size; /* default 256 */
-  int64_t rowwise_map_block_size;   /* default 256 */
+  int64_t row_reduction_block_size; /* default 256, rounded up to whole waves */
+  int64_t rowwise_map_block_size;   /* default 256 (checked; the maps' blocks
+                                       are fixed) */
   int64_t elementwise_block_size;   /* default 256 (accepted, no op uses it) */
   int64_t wavefront_size;           /* must be 64 */
   /* Wave64 extensions (no reference counterpart). */
@@ -92,14 +96,15 @@ typedef struct sw_options {
   int64_t bsr_use_mfma;             /* BSR SpMM: 1 = MFMA tiles when the block
                                        size allows it (default), 0 = the
                                        thread-per-output kernel */
-  int64_t sddmm_lanes_per_row;      /* SDDMM: 1 = thread-per-row (reference,
-                                       default); 64 = one wave per row with
+  int64_t sddmm_lanes_per_row;      /* SDDMM: 1 = the mapping's own choice
+                                       (default); 64 = one wave per row with
                                        lanes split over the dot products */
   int64_t spmm_positions_per_lane;  /* SpMM wave-per-position: consecutive
                                        positions per lane group 1,2,4,8,16;
                                        default 4 */
-  char sddmm_mapping[32];           /* thread-per-row (reference, default) |
-                                       wave-per-row | row-tile-mfma (16-row
+  char sddmm_mapping[32];           /* thread-per-row (default: the
+                                       launch is chosen by size and mean row
+                                       length) | wave-per-row | row-tile-mfma (16-row
                                        tiles on the matrix cores; tiles whose
                                        rows do not share column structure,
                                        and kdim not in {64,128,256}, use the

@@ -7,10 +7,11 @@
 //   csr_rowwise_map  ThreadPerRowCSRRowwiseMapPattern, SparseWaveToGPU.cpp:820-878
 //   attention chain  examples/pytorch/integration/SparseAttentionToSparseWave.cpp:230-315
 //
-// Each op has the reference's thread-per-row kernel and a Wave64 kernel that
-// gives a row to a wave (lanes over positions: coalesced CSR reads and, for
-// SDDMM, coalesced reads of the dense right-hand side when a row's columns
-// are contiguous, as in block masks).
+// SDDMM: 64- and 16-row matrix-core tiles for block masks, runs of positions
+// over a transposed right-hand side where scratch memory was given, one wave
+// per row for small calls, and one thread per row for the rest.  Row
+// reductions: groups of 2 to 64 lanes per row.  Row-wise maps: cut by
+// positions.  Attention: one kernel for the whole chain where its shapes fit.
 #include "sw_device.h"
 #include "sw_internal.h"
 #include "sw_sddmm_tile64.h"

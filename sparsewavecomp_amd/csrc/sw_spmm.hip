@@ -1,7 +1,8 @@
 // sparsewave.spmm on gfx950 behind sw_spmm_csr_f32.
 //
 // Reference kernels (generated IR):
-//   thread-per-output    SparseWaveToGPU.cpp:489-558
+//   thread-per-output    SparseWaveToGPU.cpp:489-558 (here lane groups:
+//                        spmm_row_group)
 //   wave-per-row-tile    SparseWaveToGPU.cpp:1057-1256
 //   thread-per-position  PositionSpMMDecomposition.cpp:19-73 +
 //                        SparsePositionScheduling.cpp:135-194
