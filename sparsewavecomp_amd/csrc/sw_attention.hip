@@ -417,13 +417,17 @@ __global__ __launch_bounds__(256) void sddmm_positions(
   const int32_t n = (int32_t)std::min<int64_t>(kWave, nnz - first);
   // (lanes past the end repeat the last position)
   const int32_t p = (int32_t)first + std::min(l, n - 1);
-  const int32_t c = col[p];
+  // positions outside the rows (ro may be a slice of a matrix's offsets, the
+  // arrays longer than the rows): their columns are not used, their row is
+  // the first or last one, and nothing is stored
+  const bool stored = p >= ro[0] && p < ro[rows];
+  const int32_t cp = col[p];
+  const int32_t c = stored ? cp : 0;
   const float sample = val != nullptr ? ldv(val + p) : 0.0f;
-  const int fr = row_search_uniform(ro, 1u, (uint32_t)rows + 1u,
-                                    (int32_t)first);
-  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows + 1u,
+  const int fr = row_search_uniform(ro, 1u, (uint32_t)rows, (int32_t)first);
+  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows,
                                    (int32_t)first + n - 1);
-  const int32_t r = row_search_lane(ro, (uint32_t)fr + 1u, (uint32_t)lr + 2u,
+  const int32_t r = row_search_lane(ro, (uint32_t)fr + 1u, (uint32_t)lr + 1u,
                                     p);
   float mine = 0.0f;
   for (int e0 = 0; e0 < n; e0 += E * U) { // wave-uniform
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(256) void sddmm_positions(
       mine = l / E == (e0 / E) + u ? s : mine;
     }
   }
-  if (l < n)
+  if (l < n && stored)
     stv(out + p, combine_sddmm(kind, sample, mine, alpha, beta));
 }
 
@@ -631,9 +635,12 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
 #pragma unroll
   for (int n = 0; n < N; ++n)
     load_window(val, first + W * (l + kWave * n), nnz, nnz, x[n]);
-  const int fr =
-      row_search_uniform(ro, 1u, (uint32_t)rows + 1u, (int32_t)first);
-  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows + 1u,
+  // positions outside the rows (ro may be a slice of a matrix's offsets, the
+  // arrays longer than the rows) find the first or last row and are not
+  // stored
+  const int32_t base = ro[0], top = ro[rows];
+  const int fr = row_search_uniform(ro, 1u, (uint32_t)rows, (int32_t)first);
+  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows,
                                    (int32_t)last);
   const int span = lr - fr; // wave-uniform
   const bool staged = span < kMapRows;
@@ -651,7 +658,7 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
 #pragma unroll
   for (int n = 0; n < N; ++n) {
     const int64_t p0 = first + W * (l + kWave * n);
-    if (p0 >= nnz)
+    if (p0 >= top)
       break;
     int row; // relative to fr
     int32_t next;
@@ -669,7 +676,7 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
       next = win[row];
       rv = rvs[row];
     } else {
-      row = row_search_lane(ro, (uint32_t)fr + 1u, (uint32_t)lr + 2u,
+      row = row_search_lane(ro, (uint32_t)fr + 1u, (uint32_t)lr + 1u,
                             (int32_t)p0) -
             fr;
       next = ro[fr + row + 1];
@@ -678,7 +685,7 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
     T y[W];
 #pragma unroll
     for (int u = 0; u < W; ++u) {
-      // (row < span also ends the walk past nnz)
+      // (row < span also ends the walk past the last row)
       while (p0 + u >= next && row < span) {
         ++row;
         next = staged ? win[row] : ro[fr + row + 1];
@@ -686,12 +693,12 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
       }
       stv(&y[u], map_value(KIND, tof(x[n][u]), rv));
     }
-    if (p0 + W <= nnz) {
+    if (p0 >= base && p0 + W <= top) {
       __builtin_memcpy(out + p0, y, sizeof y);
     } else {
 #pragma unroll
       for (int u = 0; u < W; ++u)
-        if (p0 + u < nnz)
+        if (p0 + u >= base && p0 + u < top)
           out[p0 + u] = y[u];
     }
   }

@@ -115,3 +115,37 @@ def test_map(dev, kind, copies, offset, in_place, dt):
         if dt == torch.bfloat16:
             tol = tol + 2.0 ** -8 * np.abs(want)
         assert np.all(np.abs(out.double().cpu().numpy() - want) <= tol)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,mean", [(3001, 5), (200003, 24)])
+@pytest.mark.parametrize("first,last", [(0, 1.0), (0.4, 0.4), (0.3, 0.7),
+                                        (0.999, 1.0)])
+def test_rows_that_are_a_slice(dev, first, last, rows, mean, dt):
+    """Row offsets that begin past position 0 or end before the arrays do (a
+    slice of a matrix's rows, arrays with room): entries outside the rows
+    stay as they are, the others are those of the whole matrix, bit for
+    bit."""
+    g = torch.Generator(device=G.DEV).manual_seed(rows)
+    lens = torch.randint(0, 2 * mean + 1, (rows,), generator=g, device=G.DEV)
+    ro = torch.zeros(rows + 1, dtype=torch.int32, device=G.DEV)
+    ro[1:] = torch.cumsum(lens, 0)
+    nnz = int(ro[-1])
+    val = torch.randn(nnz + 1000, generator=g, device=G.DEV).to(dt)
+    rowv = (torch.rand(rows, generator=g, device=G.DEV) + 0.5).to(dt)
+    whole = torch.empty_like(val[:nnz])
+    sw.csr_rowwise_map(ro, None, val[:nnz].clone(), rowv, whole, sw.MAP_SUB)
+    a, b = int(first * rows), max(int(last * rows), int(first * rows) + 1)
+    lo, hi = int(ro[a]), int(ro[b])
+    G.say(f"row map over rows {a}..{b} of {rows} {dt}")
+    out = torch.full_like(val, 7.0)
+    sw.csr_rowwise_map(ro[a:b + 1], None, val, rowv[a:b], out, sw.MAP_SUB)
+    red = torch.empty(b - a, dtype=dt, device=G.DEV)
+    sw.csr_row_reduce(ro[a:b + 1], None, val, red, "max")
+    torch.cuda.synchronize()
+    want = torch.full_like(val, 7.0)
+    want[lo:hi] = whole[lo:hi]
+    assert torch.equal(out, want)
+    rmax = torch.full((rows,), -float("inf"), device=G.DEV).index_reduce(
+        0, torch.repeat_interleave(lens), val[:nnz].float(), "amax")
+    assert torch.equal(red.float(), rmax[a:b])

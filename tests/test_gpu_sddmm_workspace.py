@@ -138,6 +138,36 @@ def test_block_mask_without_options(dev, orc, kdim, in_place, dt):
     _check(orc, csr, got, sw.SDDMM_AFFINE, dt, ops)
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("a,b", [(0, 40001), (9000, 40001), (9001, 31003)])
+def test_rows_that_are_a_slice(dev, a, b, dt):
+    """Row offsets that begin past position 0 or end before the arrays do:
+    entries outside the rows stay as they are, the others are those of the
+    whole matrix, bit for bit."""
+    csr = _csr(40001, 2999, 9)
+    g = torch.Generator(device=G.DEV).manual_seed(2)
+    lhs = torch.randn((csr.rows, 62), generator=g, device=G.DEV).to(dt)
+    rhs = torch.randn((62, csr.cols), generator=g, device=G.DEV).to(dt)
+    ro = G.t(csr.row_offsets)
+    # room past the rows (with columns of the matrix)
+    col = torch.cat([G.t(csr.column_indices), torch.zeros(
+        1001, dtype=torch.int32, device=G.DEV)])
+    val = torch.randn(col.numel(), generator=g, device=G.DEV).to(dt)
+    n = csr.nnz
+    lib, o = sw.load_library(), sw.Options()
+    assert lib.sw_sddmm_workspace_bytes(b - a, csr.cols, col.numel(), 62,
+                                        val.element_size(), o.ref) > 0
+    G.say(f"sddmm over rows {a}..{b} {dt}")
+    whole = sw.sddmm(ro, col[:n], val[:n], lhs, rhs, torch.empty_like(val[:n]))
+    out = torch.full_like(val, 7.0)
+    sw.sddmm(ro[a:b + 1], col, val, lhs[a:b].contiguous(), rhs, out)
+    torch.cuda.synchronize()
+    lo, hi = int(ro[a]), int(ro[b])
+    want = torch.full_like(val, 7.0)
+    want[lo:hi] = whole[lo:hi]
+    assert torch.equal(out, want)
+
+
 def test_python_call_on_another_stream_and_captured(dev, orc):
     """sw.sddmm on a side stream takes its scratch memory there; a captured
     call takes none.  Both equal the plain call's values."""
