@@ -303,15 +303,17 @@ def _fn(base, dtype, suffix=""):
 def _workspace(nbytes, like, stream):
     """Scratch memory for one call on `stream`, from torch's allocator (which
     gives it again only to later work on that stream), or None where there
-    is none to be had: under graph capture, on a stream that is not torch's,
-    or out of memory."""
+    is none to be had: under graph capture, on a stream that is not torch's or
+    of another device than the operands' (whose current stream the memory
+    would go back to under the kernel), or out of memory."""
     torch = _torch or _load_torch()
     if stream is not None:
         if not isinstance(stream, torch.cuda.Stream):
             return None
         with torch.cuda.stream(stream):
             return _workspace(nbytes, like, None)
-    if torch.cuda.is_current_stream_capturing():
+    if (like.device.index != torch.cuda.current_device()
+            or torch.cuda.is_current_stream_capturing()):
         return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
