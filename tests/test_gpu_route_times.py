@@ -1,0 +1,64 @@
+"""Calls whose shape decides between kernels, or what a kernel walks, are not
+slower than the plain alternative: each test times two public calls on the
+same operands (or on operands of the same size) and checks both results.
+
+The bars are wide (the faults they were written for were 1.5 to 1,000 times
+over them) and times are the best of several batches, so that neighbours on
+the host do not decide."""
+import numpy as np
+import pytest
+import torch
+
+import sparsewavecomp_amd as sw
+from tests import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+
+def us(fn, batches=9):
+    """Microseconds per call: the best batch, each a few calls long."""
+    for _ in range(2):
+        fn()
+    torch.cuda.synchronize()
+    best = float("inf")
+    for _ in range(batches):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(5):
+            fn()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 200.0)
+    return best
+
+
+def offsets(lens):
+    ro = torch.zeros(lens.numel() + 1, dtype=torch.int64)
+    ro[1:] = torch.cumsum(lens, 0)
+    return ro.int().to(G.DEV)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [100, 20000])
+def test_row_map_over_a_run_of_empty_rows(dev, rows, dt):
+    """100,000 empty rows between the entries of one lane's window cost a
+    search, not a walk."""
+    full = torch.full((5000,), 10, dtype=torch.int64)
+    full[-1] = 11  # the run begins inside a 16-byte window
+    lens = torch.cat([full, torch.zeros(100000, dtype=torch.int64),
+                      torch.full((rows,), 1 + 9 * (rows < 5000))])
+    ro, near = offsets(lens), offsets(lens[lens > 0])
+    val = torch.randn(int(ro[-1]), device=G.DEV).to(dt)
+    rv = torch.randn(lens.numel(), device=G.DEV).to(dt)
+    some = rv[lens.to(G.DEV) > 0]
+    out, want = torch.empty_like(val), torch.empty_like(val)
+    G.say(f"row map, run of empty rows, {rows} after it, {dt}")
+    sw.csr_rowwise_map(ro, None, val, rv, out, sw.MAP_SUB)
+    sw.csr_rowwise_map(near, None, val, some, want, sw.MAP_SUB)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    gap = us(lambda: sw.csr_rowwise_map(ro, None, val, rv, out, sw.MAP_SUB))
+    plain = us(lambda: sw.csr_rowwise_map(near, None, val, some, want,
+                                          sw.MAP_SUB))
+    print(f"run {gap:.1f} us, none {plain:.1f} us")
+    assert gap <= 6 * plain
