@@ -434,8 +434,12 @@ __global__ __launch_bounds__(256) void sddmm_positions(
   const int32_t p = (int32_t)first + std::min(l, n - 1);
   // positions outside the rows (ro may be a slice of a matrix's offsets, the
   // arrays longer than the rows): their columns are not used, their row is
-  // the first or last one, and nothing is stored
-  const bool stored = p >= ro[0] && p < ro[rows];
+  // the first or last one, and nothing is stored; a wave that holds no other
+  // ends here, so that a slice costs its own entries
+  const int32_t base = ro[0], top = ro[rows];
+  if (first >= top || first + n <= base)
+    return; // wave-uniform
+  const bool stored = p >= base && p < top;
   const int32_t cp = col[p];
   const int32_t c = stored ? cp : 0;
   const float sample = val != nullptr ? ldv(val + p) : 0.0f;
@@ -647,14 +651,17 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
   if (first >= nnz)
     return; // wave-uniform; the kernel has no workgroup barrier
   const int64_t last = std::min<int64_t>(first + kWave * W * N, nnz) - 1;
+  // positions outside the rows (ro may be a slice of a matrix's offsets, the
+  // arrays longer than the rows) find the first or last row and are not
+  // stored; a wave that holds no other ends here, so that a slice costs its
+  // own entries (2,000 of 2,000,000 rows of 20, fp32: 31 us otherwise, 9 so)
+  const int32_t base = ro[0], top = ro[rows];
+  if (first >= top || last < base)
+    return; // wave-uniform
   T x[N][W];
 #pragma unroll
   for (int n = 0; n < N; ++n)
     load_window(val, first + W * (l + kWave * n), nnz, nnz, x[n]);
-  // positions outside the rows (ro may be a slice of a matrix's offsets, the
-  // arrays longer than the rows) find the first or last row and are not
-  // stored
-  const int32_t base = ro[0], top = ro[rows];
   const int fr = row_search_uniform(ro, 1u, (uint32_t)rows, (int32_t)first);
   const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows,
                                    (int32_t)last);

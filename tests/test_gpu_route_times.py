@@ -62,3 +62,54 @@ def test_row_map_over_a_run_of_empty_rows(dev, rows, dt):
                                           sw.MAP_SUB))
     print(f"run {gap:.1f} us, none {plain:.1f} us")
     assert gap <= 6 * plain
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_row_map_of_a_slice_of_rows(dev, dt):
+    """2,000 of 2,000,000 rows cost far less than all of them."""
+    rows, mean = 2000000, 20
+    ro = (torch.arange(rows + 1, device=G.DEV) * mean).int()
+    val = torch.randn(rows * mean, device=G.DEV).to(dt)
+    rv = torch.randn(rows, device=G.DEV).to(dt)
+    out = torch.zeros_like(val)
+    a, b = 1000000, 1002000
+    G.say(f"row map of a slice {dt}")
+    part = us(lambda: sw.csr_rowwise_map(ro[a:b + 1], None, val, rv[a:b],
+                                         out, sw.MAP_SUB))
+    whole = torch.empty_like(val)
+    full = us(lambda: sw.csr_rowwise_map(ro, None, val, rv, whole,
+                                         sw.MAP_SUB))
+    lo, hi = a * mean, b * mean
+    assert torch.equal(out[lo:hi], whole[lo:hi])
+    assert not out[:lo].any() and not out[hi:].any()
+    print(f"slice {part:.1f} us, all {full:.1f} us")
+    assert part <= 0.25 * full
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_sddmm_of_a_slice_of_rows(dev, dt):
+    """A slice costs its share of the entries (and the transposition of rhs),
+    not those before it too."""
+    rows, mean, kdim, cols = 320000, 16, 96, 20000
+    g = torch.Generator(device=G.DEV).manual_seed(1)
+    ro = (torch.arange(rows + 1, device=G.DEV) * mean).int()
+    col = torch.randint(0, cols, (rows * mean,), generator=g,
+                        device=G.DEV).int()
+    val = torch.randn(rows * mean, generator=g, device=G.DEV).to(dt)
+    lhs = torch.randn((rows, kdim), generator=g, device=G.DEV).to(dt)
+    rhs = torch.randn((kdim, cols), generator=g, device=G.DEV).to(dt)
+    out, whole = torch.zeros_like(val), torch.empty_like(val)
+    a, b = 100000, 160000
+    # (the arrays end where the rows' mean is still a graph's)
+    n = ro[b].item()
+    part_ro = ro[a:b + 1]
+    some = lhs[a:b].contiguous()
+    G.say(f"sddmm of a slice {dt}")
+    part = us(lambda: sw.sddmm(part_ro, col[:n], val[:n], some, rhs, out[:n]))
+    full = us(lambda: sw.sddmm(ro, col, val, lhs, rhs, whole))
+    lo = a * mean
+    assert torch.equal(out[lo:n], whole[lo:n])
+    assert not out[:lo].any() and not out[n:].any()
+    rate = (n - lo) / whole.numel()
+    print(f"slice {part:.1f} us, all {full:.1f} us, entries {rate:.3f}")
+    assert part <= (rate + 0.2) * full
