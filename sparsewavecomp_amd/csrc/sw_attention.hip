@@ -2493,23 +2493,35 @@ bool sddmm_tiles(int64_t rows, int64_t nnz, int64_t kdim,
          ((kdim == 64 || kdim == 128) && block_rows(rows, nnz));
 }
 
-// Below this many multiply-adds a call is bound by its launches: one wave per
-// row without preparation (1,000 rows of 10, kdim = 16: 9.2 us against 17 with
-// the transposition, 30 one thread per row; 2,000 rows of 32, kdim = 96,
-// 6.2 M: 15.2 / 17.6 / 85; 4,096 rows of 90, kdim = 64, 24 M: 50 / 17.7 /
-// 587).
-bool small_sddmm(int64_t nnz, int64_t kdim) { return nnz < 8000000 / kdim; }
+// Below this many multiply-adds a call is bound by its launches.
+bool few_products(int64_t nnz, int64_t kdim) { return nnz < 8000000 / kdim; }
+
+// Few products in few rows: one wave per row without preparation (us, fp32;
+// thread per row / wave / transposed: 10,000 rows of 8, kdim = 16 29.7 / 10.5 /
+// 14.1; 30,000 of 8, kdim = 4 11.1 / 9.1 / 14.1; 60,000 of 8, kdim = 16 56 /
+// 48 / 19.5).  A wave per row costs with the rows, whatever they hold, a
+// thread per row with the longest row: 1,000,000 rows of one, kdim = 4 88 /
+// 302 / 28; 60,000 of 3, kdim = 8 13 / 23 / 14.
+bool small_sddmm(int64_t rows, int64_t nnz, int64_t kdim) {
+  return few_products(nnz, kdim) &&
+         (rows <= 16384 || (rows <= 32768 && nnz / 8 >= rows) ||
+          (rows <= 65536 && kdim >= 16));
+}
 
 // Bytes of scratch memory with which launch_sddmm transposes rhs first (0:
 // it would not).  A transposition reads and writes rhs once, a gathered
 // column costs a line per element: worth it from one entry per four columns
 // on, and not for block masks, whose gathers share their lines (8,192 rows of
-// 345 entries, kdim = 96: 71 us one wave per row, 94 transposed).  At most
-// 1 GiB.
+// 345 entries, kdim = 96: 71 us one wave per row, 94 transposed).  Few
+// products are worth it from 500,000 elements of lhs on (30,000 rows of 3,
+// kdim = 32 52 us one wave per row, 15.3 transposed; 30,000 of 8, kdim = 4 9.1
+// and 14.1), except the single product of kdim = 1 (1,000,000 rows of 3 41 us
+// one thread per row, 53 transposed).  At most 1 GiB.
 int64_t sddmm_workspace(int64_t rows, int64_t cols, int64_t nnz, int64_t kdim,
                         int64_t elem, const sw_options &o) {
   if (rows <= 0 || cols <= 0 || kdim <= 0 || kdim > INT32_MAX / 2 ||
-      small_sddmm(nnz, kdim) || nnz < cols / 4 || block_rows(rows, nnz) ||
+      (few_products(nnz, kdim) && (kdim == 1 || rows < 500000 / kdim)) ||
+      nnz < cols / 4 || block_rows(rows, nnz) ||
       (streq(o.sddmm_mapping, "row-tile-mfma") &&
        (kdim == 64 || kdim == 128 || kdim == 256)))
     return 0;
@@ -2669,12 +2681,13 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
       return launch_check("SDDMM tile MFMA kernel");
     }
   }
-  // (thread-per-row: only many short rows without scratch memory; rows of a
+  // (thread-per-row: many short rows without scratch memory; rows of a
   // block mask past its kernels' kdim, 8,192 of 345 entries, kdim = 96, take
   // 562 us one thread per row, 71 one wave)
   if (streq(o.sddmm_mapping, "wave-per-row") ||
       (streq(o.sddmm_mapping, "row-tile-mfma")) ||
-      o.sddmm_lanes_per_row == 64 || small_sddmm(nnz, std::max<int64_t>(kdim, 1)) ||
+      o.sddmm_lanes_per_row == 64 ||
+      small_sddmm(rows, nnz, std::max<int64_t>(kdim, 1)) ||
       block_rows(rows, nnz)) {
     int rc = grid_for(rows, 4, "SDDMM", &grid);
     if (rc)
