@@ -2484,13 +2484,24 @@ bool long_rows(int64_t rows, int64_t nnz) { return nnz / 400 > rows; }
 // row 645.)
 bool block_rows(int64_t rows, int64_t nnz) { return nnz / 96 >= rows; }
 
+// One wave per row was asked for.  (With scratch memory the rhs is transposed
+// all the same: 44.5 us against 643 for the graph below.)
+bool asks_wave(const sw_options &o) {
+  return streq(o.sddmm_mapping, "wave-per-row") ||
+         (o.sddmm_lanes_per_row == 64 &&
+          !streq(o.sddmm_mapping, "row-tile-mfma"));
+}
+
 // The 16-row tiles of the fused attention kernel's product phase serve this
-// call: asked for, or rows long enough.  (kdim 256 and bf16's or fp32's other
+// call: asked for, or rows long enough and no wave per row asked for (rows
+// that share no columns gain nothing from a tile: 100 rows of 1,000 random
+// columns of 2,000, kdim = 64, 41 us one wave per row, 124 in tiles).  (kdim 256 and bf16's or fp32's other
 // tile kernels are chosen in launch_sddmm.)
 bool sddmm_tiles(int64_t rows, int64_t nnz, int64_t kdim,
                  const sw_options &o) {
   return streq(o.sddmm_mapping, "row-tile-mfma") ||
-         ((kdim == 64 || kdim == 128) && block_rows(rows, nnz));
+         ((kdim == 64 || kdim == 128) && block_rows(rows, nnz) &&
+          !asks_wave(o));
 }
 
 // Below this many multiply-adds a call is bound by its launches.
@@ -2684,9 +2695,7 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
   // (thread-per-row: many short rows without scratch memory; rows of a
   // block mask past its kernels' kdim, 8,192 of 345 entries, kdim = 96, take
   // 562 us one thread per row, 71 one wave)
-  if (streq(o.sddmm_mapping, "wave-per-row") ||
-      (streq(o.sddmm_mapping, "row-tile-mfma")) ||
-      o.sddmm_lanes_per_row == 64 ||
+  if (asks_wave(o) || streq(o.sddmm_mapping, "row-tile-mfma") ||
       small_sddmm(rows, nnz, std::max<int64_t>(kdim, 1)) ||
       block_rows(rows, nnz)) {
     int rc = grid_for(rows, 4, "SDDMM", &grid);

@@ -157,3 +157,29 @@ def test_sddmm_of_many_short_rows(dev, rows, mean, kdim, dt):
     print(f"default {call:.1f} us, without scratch {alone:.1f} us, "
           f"wave {wave:.1f} us")
     assert max(call, alone) <= 0.6 * wave
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("options", ["sddmm-mapping=wave-per-row",
+                                     "sddmm-lanes-per-row=64"])
+def test_sddmm_wave_per_row_of_long_rows(dev, options, dt):
+    """A wave per row that is asked for is one, where rows long enough for the
+    16-row tiles share no columns."""
+    g = torch.Generator(device=G.DEV).manual_seed(1)
+    rows, cols, mean, kdim = 100, 2000, 1000, 64
+    ro = (torch.arange(rows + 1, device=G.DEV) * mean).int()
+    col = torch.rand((rows, cols), generator=g, device=G.DEV).argsort(
+        1)[:, :mean].sort(1).values.int().reshape(-1)
+    val = torch.randn(rows * mean, generator=g, device=G.DEV).to(dt)
+    lhs = torch.randn((rows, kdim), generator=g, device=G.DEV).to(dt)
+    rhs = torch.randn((kdim, cols), generator=g, device=G.DEV).to(dt)
+    out, want = torch.empty_like(val), torch.empty_like(val)
+    G.say(f"sddmm wave per row {dt} {options}")
+    o = sw.Options.parse(options)
+    wave = us(lambda: sw.sddmm(ro, col, val, lhs, rhs, out, options=o))
+    tiles = us(lambda: sw.sddmm(ro, col, val, lhs, rhs, want))
+    # (both sum 64 products in fp32)
+    assert float((out.float() - want.float()).norm()) <= (
+        2e-6 if dt == torch.float32 else 8e-3) * float(want.float().norm())
+    print(f"asked {wave:.1f} us, default {tiles:.1f} us")
+    assert wave <= 0.7 * tiles
