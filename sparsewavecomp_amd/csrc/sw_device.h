@@ -147,6 +147,15 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t b, int64_t n) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// The same with each XCD taking chunks of eight neighbours in turn, for work
+// whose weight may drift along the index (rows sorted by length): a contiguous
+// eighth of such work can hold most of it.  A bijection on [0, n); the last
+// n % 64 keep their order.
+__device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t n) {
+  const int64_t first = b & ~(int64_t)63;
+  return first + 64 <= n ? first + (b & 7) * 8 + ((b >> 3) & 7) : b;
+}
+
 // Shift by one lane up / down across the whole wave (ds_bpermute).
 __device__ __forceinline__ int shfl_up1_i(int v, int fill) {
   int l = lane_id();

@@ -183,3 +183,37 @@ def test_sddmm_wave_per_row_of_long_rows(dev, options, dt):
         2e-6 if dt == torch.float32 else 8e-3) * float(want.float().norm())
     print(f"asked {wave:.1f} us, default {tiles:.1f} us")
     assert wave <= 0.7 * tiles
+
+
+def _csr(lens, cols, dt, seed=1):
+    """Row offsets, random columns and values of rows of these lengths."""
+    g = torch.Generator(device=G.DEV).manual_seed(seed)
+    ro = offsets(lens)
+    n = int(ro[-1])
+    col = torch.randint(0, cols, (n,), generator=g, device=G.DEV).int()
+    return ro, col, torch.rand(n, generator=g, device=G.DEV).to(dt)
+
+
+def _spmm_call(lens, k, dt, options=None, cols=100000):
+    ro, col, val = _csr(lens, cols, dt)
+    g = torch.Generator(device=G.DEV).manual_seed(2)
+    rhs = torch.rand((cols, k), generator=g, device=G.DEV).to(dt)
+    out = torch.empty((lens.numel(), k), dtype=dt, device=G.DEV)
+    o = sw.Options.parse(options) if options else None
+    return lambda: sw.spmm(ro, col, val, rhs, out, options=o)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_spmm_of_rows_sorted_by_length(dev, dt):
+    """Rows sorted by their lengths are spread over the chip as shuffled ones
+    are."""
+    g = torch.Generator().manual_seed(3)
+    lens = torch.exp(1.5 * torch.randn(200000, generator=g) + 1.9)
+    lens = lens.round().clamp(1, 4096).long()
+    G.say(f"spmm of sorted rows {dt}")
+    mixed = us(_spmm_call(lens, 100, dt))
+    up = us(_spmm_call(lens.sort().values, 100, dt))
+    down = us(_spmm_call(lens.sort(descending=True).values, 100, dt))
+    print(f"ascending {up:.1f} us, descending {down:.1f} us, "
+          f"shuffled {mixed:.1f} us")
+    assert max(up, down) <= 1.8 * mixed
