@@ -918,12 +918,23 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
   // mean of 48 entries more of them in flight are worth more than whole
   // rows of rhs at once (fp32, 100,000 rows of 60, k = 128, CL 8 / 16 / 32:
   // 464 / 531 / 618 us, k = 33 221 / 274; 200,003 rows of 20, k = 100 302 /
-  // 288 / 320).  PL entries at a time: 4 below a mean of 32 (k = 16, bf16,
-  // PL 4 / 16: rows of 20 43 / 50 us, of 60 57 / 52).
+  // 288 / 320).
   const int V = k >= 8 && sizeof(T) == 2 ? 8 : k >= 4 ? 4 : k >= 2 ? 2 : 1;
   const int CL = next_pow2((int)std::min<int64_t>(
       ceil_div(k, V), nnz / 48 >= rows ? 8 : 16));
-  const int G = std::min(64, CL * (nnz / 32 < rows ? 4 : 16));
+  // PL entries at a time, by the mean row: lanes past a row's entries still
+  // take part in its steps and its butterfly.  us, fp32, PL 1 / 2 / 4:
+  // 1,000,000 rows of 0.05 entries k = 64 60 / 81 / 132, of 2 108 / 141 / 258,
+  // of 4 159 / 176 / 268 (one thread per output 105, 210, 242); 500,000 of 8
+  // 143 / 137 / 152 (145), k = 1 27 / 23 / 20 (19); k = 16, bf16, PL 4 / 16:
+  // rows of 20 43 / 50, of 32 39 / 45, of 60 41 / 33.  From 3 entries on not
+  // 1: rows sorted by length (1,000,000 of 4, k = 64) 420 / 358, 344 one
+  // thread per output.
+  const int PL = nnz / 3 < rows    ? 1
+                 : nnz / 12 < rows ? (CL == 1 ? 4 : 2)
+                 : nnz / 48 < rows ? 4
+                                   : 16;
+  const int G = std::min(64, CL * PL);
   const int64_t tiles = ceil_div(k, (int64_t)CL * V);
   const int64_t grid =
       std::max<int64_t>(ceil_div(rows * tiles, 256 / G), 1);
@@ -932,23 +943,41 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
     return rc;
   const dim3 g = grid_dim(grid, 256);
 #define SW_ROWS(VV, CC, GG)                                                   \
-  if (V == VV && CL == CC && G == GG)                                         \
-  hipLaunchKernelGGL((spmm_row_group<T, VV, CC, GG>), g, dim3(256), 0, st,  \
-                     ro, col, val, rhs, out, rows, k, tiles);
-#define SW_ROWS_V(VV)                                                         \
-  SW_ROWS(VV, 1, 4) SW_ROWS(VV, 1, 16) SW_ROWS(VV, 2, 8) SW_ROWS(VV, 2, 32)   \
-  SW_ROWS(VV, 4, 16) SW_ROWS(VV, 4, 64) SW_ROWS(VV, 8, 32)                    \
-  SW_ROWS(VV, 8, 64) SW_ROWS(VV, 16, 64)
+  case VV * 10000 + CC * 100 + GG:                                            \
+    hipLaunchKernelGGL((spmm_row_group<T, VV, CC, GG>), g, dim3(256), 0, st,  \
+                       ro, col, val, rhs, out, rows, k, tiles);               \
+    break;
+#define SW_ROWS_1(VV) SW_ROWS(VV, 1, 1) SW_ROWS(VV, 1, 4) SW_ROWS(VV, 1, 16)
+#define SW_ROWS_2(VV)                                                         \
+  SW_ROWS_1(VV) SW_ROWS(VV, 2, 2) SW_ROWS(VV, 2, 4) SW_ROWS(VV, 2, 8)         \
+  SW_ROWS(VV, 2, 32)
+#define SW_ROWS_16(VV)                                                        \
+  SW_ROWS_2(VV) SW_ROWS(VV, 4, 4) SW_ROWS(VV, 4, 8) SW_ROWS(VV, 4, 16)        \
+  SW_ROWS(VV, 4, 64) SW_ROWS(VV, 8, 8) SW_ROWS(VV, 8, 16) SW_ROWS(VV, 8, 32)  \
+  SW_ROWS(VV, 8, 64) SW_ROWS(VV, 16, 16) SW_ROWS(VV, 16, 32)                  \
+  SW_ROWS(VV, 16, 64)
+  bool known = true;
+  const int shape = V * 10000 + CL * 100 + G;
   if constexpr (sizeof(T) == 2) {
-    SW_ROWS_V(8)
-    SW_ROWS(4, 1, 4) SW_ROWS(4, 1, 16) SW_ROWS(4, 2, 8) SW_ROWS(4, 2, 32)
+    switch (shape) {
+      SW_ROWS_16(8) SW_ROWS_2(4) SW_ROWS_2(2) SW_ROWS_1(1)
+    default:
+      known = false;
+    }
   } else {
-    SW_ROWS_V(4)
+    switch (shape) {
+      SW_ROWS_16(4) SW_ROWS_2(2) SW_ROWS_1(1)
+    default:
+      known = false;
+    }
   }
-  SW_ROWS(2, 1, 4) SW_ROWS(2, 1, 16) SW_ROWS(2, 2, 8) SW_ROWS(2, 2, 32)
-  SW_ROWS(1, 1, 4) SW_ROWS(1, 1, 16)
-#undef SW_ROWS_V
+#undef SW_ROWS_16
+#undef SW_ROWS_2
+#undef SW_ROWS_1
 #undef SW_ROWS
+  if (!known)
+    return fail(SW_ERR_INVALID_SHAPE, "%s has no kernel for k = %lld", what,
+                (long long)k);
   return launch_check("SpMM row kernel");
 }
 

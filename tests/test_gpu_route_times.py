@@ -217,3 +217,30 @@ def test_spmm_of_rows_sorted_by_length(dev, dt):
     print(f"ascending {up:.1f} us, descending {down:.1f} us, "
           f"shuffled {mixed:.1f} us")
     assert max(up, down) <= 1.8 * mixed
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 33, 64])
+def test_spmm_of_nearly_empty_rows(dev, k, dt):
+    """A product of rows of which one in twenty holds an entry takes a few
+    times what writing its output does (two launches' floors, and rows of
+    k = 33 that share their lines with neighbours)."""
+    lens = (torch.arange(1000000) % 20 == 0).long()
+    out = torch.empty((1000000, k), device=G.DEV, dtype=dt)
+    G.say(f"spmm of nearly empty rows k={k} {dt}")
+    fill = us(lambda: out.fill_(1.0))
+    call = us(_spmm_call(lens, k, dt))
+    print(f"product {call:.1f} us, fill {fill:.1f} us")
+    assert call <= 3 * fill + 6
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [16, 64, 100])
+def test_spmm_of_short_rows(dev, k, dt):
+    """The same entries in rows of 4 take little longer than in rows of 16
+    (four times the output)."""
+    G.say(f"spmm of short rows k={k} {dt}")
+    short = us(_spmm_call(torch.full((1000000,), 4), k, dt))
+    long = us(_spmm_call(torch.full((250000,), 16), k, dt))
+    print(f"rows of 4 {short:.1f} us, of 16 {long:.1f} us")
+    assert short <= 1.9 * long
