@@ -919,9 +919,11 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
   // rows of rhs at once (fp32, 100,000 rows of 60, k = 128, CL 8 / 16 / 32:
   // 464 / 531 / 618 us, k = 33 221 / 274; 200,003 rows of 20, k = 100 302 /
   // 288 / 320).
-  const int V = k >= 8 && sizeof(T) == 2 ? 8 : k >= 4 ? 4 : k >= 2 ? 2 : 1;
-  const int CL = next_pow2((int)std::min<int64_t>(
-      ceil_div(k, V), nnz / 48 >= rows ? 8 : 16));
+  // From a mean of 128 on whole rows again (5,000 rows of 300, k = 100, CL 8 /
+  // 16: fp32 98 / 90, bf16 53 / 35 us).
+  int V = k >= 8 && sizeof(T) == 2 ? 8 : k >= 4 ? 4 : k >= 2 ? 2 : 1;
+  int CL = next_pow2((int)std::min<int64_t>(
+      ceil_div(k, V), nnz / 48 >= rows && nnz / 128 < rows ? 8 : 16));
   // PL entries at a time, by the mean row: lanes past a row's entries still
   // take part in its steps and its butterfly.  us, fp32, PL 1 / 2 / 4:
   // 1,000,000 rows of 0.05 entries k = 64 60 / 81 / 132, of 2 108 / 141 / 258,
@@ -934,7 +936,18 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
                  : nnz / 12 < rows ? (CL == 1 ? 4 : 2)
                  : nnz / 48 < rows ? 4
                                    : 16;
-  const int G = std::min(64, CL * PL);
+  int G = std::min(64, CL * PL);
+  // Few long rows: a wave for each, and narrower tiles of it until there are
+  // a thousand waves (20 rows of 20,000, bf16: k = 128 518 -> 84 us, k = 4
+  // 122 -> 27).
+  auto waves = [&] { return rows * ceil_div(k, (int64_t)CL * V); };
+  if (nnz / 48 >= rows && waves() * G / 64 < 2048) {
+    G = 64;
+    while (CL > 1 && waves() < 1024)
+      CL /= 2;
+    if (V == 8 && CL == 1 && waves() < 1024)
+      V = 4;
+  }
   const int64_t tiles = ceil_div(k, (int64_t)CL * V);
   const int64_t grid =
       std::max<int64_t>(ceil_div(rows * tiles, 256 / G), 1);
@@ -947,10 +960,11 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
     hipLaunchKernelGGL((spmm_row_group<T, VV, CC, GG>), g, dim3(256), 0, st,  \
                        ro, col, val, rhs, out, rows, k, tiles);               \
     break;
-#define SW_ROWS_1(VV) SW_ROWS(VV, 1, 1) SW_ROWS(VV, 1, 4) SW_ROWS(VV, 1, 16)
+#define SW_ROWS_1(VV)                                                         \
+  SW_ROWS(VV, 1, 1) SW_ROWS(VV, 1, 4) SW_ROWS(VV, 1, 16) SW_ROWS(VV, 1, 64)
 #define SW_ROWS_2(VV)                                                         \
   SW_ROWS_1(VV) SW_ROWS(VV, 2, 2) SW_ROWS(VV, 2, 4) SW_ROWS(VV, 2, 8)         \
-  SW_ROWS(VV, 2, 32)
+  SW_ROWS(VV, 2, 32) SW_ROWS(VV, 2, 64)
 #define SW_ROWS_16(VV)                                                        \
   SW_ROWS_2(VV) SW_ROWS(VV, 4, 4) SW_ROWS(VV, 4, 8) SW_ROWS(VV, 4, 16)        \
   SW_ROWS(VV, 4, 64) SW_ROWS(VV, 8, 8) SW_ROWS(VV, 8, 16) SW_ROWS(VV, 8, 32)  \

@@ -244,3 +244,39 @@ def test_spmm_of_short_rows(dev, k, dt):
     long = us(_spmm_call(torch.full((250000,), 16), k, dt))
     print(f"rows of 4 {short:.1f} us, of 16 {long:.1f} us")
     assert short <= 1.9 * long
+
+
+@pytest.mark.parametrize("k", [4, 64, 200])
+def test_spmm_of_few_long_rows(dev, k):
+    """20 rows of 20,000 entries fill the chip in bf16 as fp32's row tiles of
+    four columns do (bf16's row tiles are the kernel of calls without
+    options)."""
+    lens = torch.full((20,), 20000)
+    tile = "spmm-mapping=wave-per-row-tile"
+    G.say(f"spmm of few long rows k={k}")
+    want = us(_spmm_call(lens, k, torch.float32, tile))
+    call = us(_spmm_call(lens, k, torch.bfloat16, tile))
+    plain = us(_spmm_call(lens, k, torch.float32))
+    print(f"bf16 {call:.1f} us, fp32 {plain:.1f} us, fp32 tiles {want:.1f}")
+    assert max(call, plain) <= 1.8 * want
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,mean,k", [(3, 1500, 1), (3, 1500, 6),
+                                         (3, 1500, 130), (40, 200, 33),
+                                         (1, 5000, 8), (700, 140, 100)])
+def test_spmm_of_few_long_rows_values(dev, orc, rows, mean, k, dt):
+    """Every shape that few long rows choose, against the oracle's bound."""
+    cols = 3000
+    ro, col, val = _csr(torch.full((rows,), mean), cols, dt)
+    g = torch.Generator(device=G.DEV).manual_seed(4)
+    rhs = torch.randn((cols, k), generator=g, device=G.DEV).to(dt)
+    out = torch.full((rows, k), float("nan"), dtype=dt, device=G.DEV)
+    G.say(f"spmm of few long rows {rows} x {mean} k={k} {dt}")
+    sw.spmm(ro, col, val, rhs, out)
+    torch.cuda.synchronize()
+    host = [x.cpu().numpy() for x in (ro, col, val.float(), rhs.float())]
+    ref, bound = orc.spmm(*host), 1e-5 * orc.spmm_abs_bound(*host)
+    if dt == torch.bfloat16:  # one rounding more
+        bound = bound + 2.0 ** -8 * np.abs(ref)
+    assert np.all(np.abs(out.float().cpu().numpy() - ref) <= bound)
