@@ -929,12 +929,13 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
   // 1,000,000 rows of 0.05 entries k = 64 60 / 81 / 132, of 2 108 / 141 / 258,
   // of 4 159 / 176 / 268 (one thread per output 105, 210, 242); 500,000 of 8
   // 143 / 137 / 152 (145), k = 1 27 / 23 / 20 (19); k = 16, bf16, PL 4 / 16:
-  // rows of 20 43 / 50, of 32 39 / 45, of 60 41 / 33.  From 3 entries on not
+  // rows of 20 43 / 50, of 32 39 / 45, of 60 41 / 33 (k = 1, rows of 20 of
+  // very unequal length 26 / 24, sorted by it 122 / 56).  From 3 entries on not
   // 1: rows sorted by length (1,000,000 of 4, k = 64) 420 / 358, 344 one
   // thread per output.
   const int PL = nnz / 3 < rows    ? 1
                  : nnz / 12 < rows ? (CL == 1 ? 4 : 2)
-                 : nnz / 48 < rows ? 4
+                 : nnz / 48 < rows ? (CL == 1 ? 16 : 4)
                                    : 16;
   int G = std::min(64, CL * PL);
   // Few long rows: a wave for each, and narrower tiles of it until there are
@@ -1102,7 +1103,16 @@ bool launch_spmm_rows(const int32_t *ro, const int32_t *col, const T *val,
     const int T_ = (int)o.spmm_tile_size;
     const int64_t tpr = ceil_div(k, T_);
     const bool vec = (T_ % 4 == 0) && (k % 4 == 0) && vec_ok(rhs) && vec_ok(out);
-    const bool any = !vec && T_ % 4 == 0 && k >= 4;
+    // Four columns a lane at any alignment leave a row to four times the
+    // position lanes, whose butterfly sums four values over them: worth it
+    // from 3 entries for every 8 position lanes on (us, fp32, k = 33, one
+    // column / four: tile 4, 64 lanes rows of 4 1710 / 2163, of 8 890 / 1100,
+    // of 20 449 / 432; tile 16 rows of 4 586 / 663, of 8 305 / 290).
+    const int64_t any_lanes =
+        std::max<int64_t>(o.spmm_lanes_per_row, next_pow2(ceil_div(T_, 4))) /
+        next_pow2(ceil_div(T_, 4));
+    const bool any = !vec && T_ % 4 == 0 && k >= 4 &&
+                     nnz / (3 * any_lanes) >= rows / 8;
     const int V = vec || any ? 4 : 1;
     const int CL = next_pow2(ceil_div(T_, V));
     const int G = std::max<int>((int)o.spmm_lanes_per_row, CL);

@@ -280,3 +280,18 @@ def test_spmm_of_few_long_rows_values(dev, orc, rows, mean, k, dt):
     if dt == torch.bfloat16:  # one rounding more
         bound = bound + 2.0 ** -8 * np.abs(ref)
     assert np.all(np.abs(out.float().cpu().numpy() - ref) <= bound)
+
+
+@pytest.mark.parametrize("mean", [0, 4])
+def test_spmm_row_tile_of_short_rows_at_odd_widths(dev, mean):
+    """Narrow tiles of k = 7 keep one column a lane where rows are short: less
+    than the four columns a lane of k = 8 take.  (mean 0: an entry in one row
+    of twenty.)"""
+    lens = (torch.full((1000000,), mean) if mean else
+            (torch.arange(1000000) % 20 == 0).long())
+    tile = "spmm-mapping=wave-per-row-tile spmm-lanes-per-row=64"
+    G.say(f"spmm row tile of short rows mean={mean}")
+    odd = us(_spmm_call(lens, 7, torch.float32, tile))
+    even = us(_spmm_call(lens, 8, torch.float32, tile))
+    print(f"k = 7 {odd:.1f} us, k = 8 {even:.1f} us")
+    assert odd <= 0.85 * even
