@@ -295,3 +295,32 @@ def test_spmm_row_tile_of_short_rows_at_odd_widths(dev, mean):
     even = us(_spmm_call(lens, 8, torch.float32, tile))
     print(f"k = 7 {odd:.1f} us, k = 8 {even:.1f} us")
     assert odd <= 0.85 * even
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,mean", [(100000, 4), (200000, 0)])
+def test_attention_of_many_short_rows(dev, rows, mean, dt):
+    """Without options, many rows of a few unshared columns cost what the six
+    separate ops cost (mean 0: one entry in every tenth row)."""
+    lens = (torch.full((rows,), mean) if mean else
+            (torch.arange(rows) % 10 == 0).long())
+    ro, col, mask = _csr(lens, rows, dt)
+    g = torch.Generator(device=G.DEV).manual_seed(4)
+    q, v = (torch.randn((rows, 64), generator=g, device=G.DEV).to(dt)
+            for _ in range(2))
+    kt = torch.randn((64, rows), generator=g, device=G.DEV).to(dt)
+
+    def call(options):
+        s, m, r = (torch.empty(n, device=G.DEV, dtype=dt)
+                   for n in (col.numel(), rows, rows))
+        out = torch.empty((rows, 64), device=G.DEV, dtype=dt)
+        o = sw.Options.parse(options) if options else None
+        return lambda: sw.sparse_attention(ro, col, mask, q, kt, v, s, m, r,
+                                           out, 0.125, 1.0, options=o)
+
+    G.say(f"attention of many short rows {rows} x {mean} {dt}")
+    # (any block size that is not the default asks for the separate ops)
+    six = us(call("rowwise-map-block-size=128"))
+    plain = us(call(None))
+    print(f"default {plain:.1f} us, six ops {six:.1f} us")
+    assert plain <= 1.2 * six
