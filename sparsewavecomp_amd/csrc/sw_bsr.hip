@@ -621,12 +621,37 @@ int check_bsr(const int32_t *bro, const int32_t *bcol, const void *bval,
 constexpr int kBf16Batch = 1;
 constexpr int kBf16Split = 4;
 
+// Few products per block row: thread-per-output is faster than a 16-row tile
+// per block row, whose waves cost the same however little of it b and k fill.
+// In products (b rows of k outputs of `entries` terms each, and about four
+// terms' worth of addressing).  Sweeps over 131,072 and 524,288 rows, thread
+// per output / bsr_mfma, us: fp32 4 x 4 blocks, one a block row, k = 1 9 / 101,
+// k = 16 42 / 89, k = 32 84 / 88; six 31 / 143, 152 / 126 (k = 16); 8 x 8, one,
+// k = 8 30 / 46, k = 16 57 / 47; 12 x 12, one, k = 4 20 / 32, k = 8 38 / 32;
+// 20 x 20, one, k = 8 54 / 64, k = 16 104 / 65, three, k = 1 25 / 27.  bf16
+// 4 x 4, one, k = 24 61 / 66, k = 32 78 / 66; 8 x 8, six, k = 2 36 / 55, k = 4
+// 63 / 51; 12 x 12, six, k = 1 56 / 46; 20 x 20, one, k = 2 19 / 26, k = 4
+// 24 / 23.  (16 x 16 blocks always take the matrix cores.)
+template <typename T>
+bool few_block_products(int64_t b, double entries, int64_t k) {
+  const double products = (double)b * (double)k * (entries + 4.0);
+  if (b == 16 || b >= 32)
+    return false;
+  if (sizeof(T) == 2)
+    return products < 950.0;
+  return b < 16 ? products < 1000.0 + 25.0 * entries
+                : products < 4300.0 && entries <= 40.0;
+}
+
 template <typename T, typename TO>
 int launch_bsr(const int32_t *bro, const int32_t *bcol, const T *bval,
-               const T *rhs, TO *out, int64_t rows, int64_t cols, int64_t k,
-               int64_t b, const sw_options &o, hipStream_t st, bool mfma) {
+               const T *rhs, TO *out, int64_t rows, int64_t cols, int64_t nnzb,
+               int64_t k, int64_t b, const sw_options &o, hipStream_t st,
+               bool mfma) {
   if (rows == 0 || k == 0)
     return SW_OK;
+  mfma = mfma && !few_block_products<T>(
+                     b, (double)nnzb * (double)(b * b) / (double)rows, k);
   const int nbr = (int)(rows / 16);
   // The matrix-core kernels' x must stay within one grid dimension's
   // 2^32 - 1 work-items; past it the thread-per-output kernel below, whose
@@ -761,7 +786,7 @@ int bsr_entry(const int32_t *block_row_offsets,
   if (rc)
     return rc;
   return launch_bsr<T, TO>(block_row_offsets, block_column_indices,
-                           block_values, rhs, output, rows, cols, k,
+                           block_values, rhs, output, rows, cols, nnzb, k,
                            block_size, o, sw::as_stream(stream),
                            o.bsr_use_mfma != 0);
 }

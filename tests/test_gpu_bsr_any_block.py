@@ -40,7 +40,8 @@ def _at(a, dtype, offset):
 
 
 @pytest.mark.parametrize("offset", [0, 1])
-@pytest.mark.parametrize("b,k", [(4, 1), (4, 64), (4, 130), (8, 7), (8, 200),
+@pytest.mark.parametrize("b,k", [(4, 1), (4, 33), (4, 64), (4, 130), (8, 7),
+                                 (8, 200), (12, 5),
                                  (12, 61), (16, 64), (16, 65), (16, 30),
                                  (16, 200), (20, 8), (32, 3), (32, 100),
                                  (32, 264), (40, 129), (48, 64), (64, 200),

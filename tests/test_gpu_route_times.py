@@ -324,3 +324,29 @@ def test_attention_of_many_short_rows(dev, rows, mean, dt):
     plain = us(call(None))
     print(f"default {plain:.1f} us, six ops {six:.1f} us")
     assert plain <= 1.2 * six
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,k,blocks", [(4, 1, 1), (4, 4, 6), (8, 4, 1),
+                                        (12, 2, 1), (20, 1, 1), (4, 16, 1)])
+def test_bsr_of_few_products(dev, b, k, blocks, dt):
+    """Narrow products of small blocks are not slower than one thread per
+    output."""
+    nbr = 524288 // b
+    g = torch.Generator(device=G.DEV).manual_seed(5)
+    ro = (torch.arange(nbr + 1, device=G.DEV) * blocks).int()
+    col = torch.randint(0, nbr, (nbr * blocks,), generator=g,
+                        device=G.DEV).int()
+    val = torch.randn((nbr * blocks, b, b), generator=g, device=G.DEV).to(dt)
+    rhs = torch.randn((nbr * b, k), generator=g, device=G.DEV).to(dt)
+    out, want = (torch.empty((nbr * b, k), device=G.DEV, dtype=dt)
+                 for _ in range(2))
+    o = sw.Options.parse("bsr-use-mfma=0")
+    G.say(f"bsr of few products b={b} k={k} blocks={blocks} {dt}")
+    call = us(lambda: sw.bsr_spmm(ro, col, val, rhs, out, b))
+    plain = us(lambda: sw.bsr_spmm(ro, col, val, rhs, want, b, options=o))
+    # (sums of up to 24 products in another order)
+    assert float((out.float() - want.float()).norm()) <= (
+        2e-6 if dt == torch.float32 else 8e-3) * float(want.float().norm())
+    print(f"default {call:.1f} us, thread per output {plain:.1f} us")
+    assert call <= 1.25 * plain
