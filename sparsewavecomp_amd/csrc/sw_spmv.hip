@@ -1167,9 +1167,12 @@ int launch_spmv_coo(const int32_t *ri, const int32_t *col, const float *val,
   // 39 / 32 / 32 us, 1,000,000 rows of 20: 131 / 160 / 128 / 130 us, against
   // 300 and 1235 us with one thread and one atomic add per entry; shuffled
   // entries (every run one entry) 250 and 981 us either way.
+  // Below two entries a row one too: a lane's runs are then one entry each, and
+  // four of them go out as four adds of every fourth element (1,000,000 rows of
+  // one entry: P = 1 / 4 13.0 / 19.5 us, of two 19.5 / 19.5).
   const int64_t P = streq(o.spmv_mapping, "wave-per-position")
                         ? o.spmv_positions_per_lane
-                        : (vec ? 4 : 1);
+                        : (vec && nnz / 2 >= rows ? 4 : 1);
   // whole waves (spmv-block-size may be any size outside the position
   // mapping)
   const int64_t RB = ceil_div(B, kWave) * kWave;

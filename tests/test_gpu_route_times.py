@@ -350,3 +350,28 @@ def test_bsr_of_few_products(dev, b, k, blocks, dt):
         2e-6 if dt == torch.float32 else 8e-3) * float(want.float().norm())
     print(f"default {call:.1f} us, thread per output {plain:.1f} us")
     assert call <= 1.25 * plain
+
+
+def test_coo_of_one_entry_a_row(dev):
+    """Aligned arrays of sorted entries, one a row, are not slower than the
+    same off their alignment (one entry a lane)."""
+    n = 1000000
+    g = torch.Generator(device=G.DEV).manual_seed(6)
+    ri = torch.arange(n + 4, device=G.DEV).int()
+    col = torch.randint(0, n, (n + 4,), generator=g, device=G.DEV).int()
+    val = torch.rand(n + 4, generator=g, device=G.DEV)
+    x = torch.rand(n, generator=g, device=G.DEV)
+    y = torch.empty(n + 4, device=G.DEV)
+    G.say("coo, one entry a row")
+
+    def call(a, z):
+        return lambda: sw.coo_spmv(ri[a:z], col[a:z], val[a:z], x, y)
+
+    even = us(call(0, n))
+    sums = y.clone()
+    odd = us(call(1, n + 1))
+    # one product a row either way
+    assert torch.equal(sums[1:n], y[1:n])
+    assert torch.equal(sums[:n], val[:n] * x[col[:n].long()])
+    print(f"aligned {even:.1f} us, off by one {odd:.1f} us")
+    assert even <= 1.25 * odd
