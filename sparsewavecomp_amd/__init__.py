@@ -519,8 +519,11 @@ def sddmm(row_offsets, column_indices, values, lhs, rhs, output_values,
             _dev(rhs, dt, "rhs"), _dev(output_values, dt, "output_values"),
             rows, rhs.shape[1], nnz, lhs.shape[1], combine, alpha, beta,
             _opts(options))
-    need = load_library().sw_sddmm_workspace_bytes(
-        *args[6:10], output_values.element_size(), args[-1])
+    need, k = 0, lhs.shape[1]
+    if rows * k >= 500000 or nnz * k >= 8000000:
+        # (below both the answer is 0, and asking takes 1 us of a call's 9)
+        need = load_library().sw_sddmm_workspace_bytes(
+            *args[6:10], output_values.element_size(), args[-1])
     workspace = _workspace(need, rhs, stream) if need > 0 else None
     if workspace is None:
         _check(_fn("sw_sddmm_csr", dt)(*args, _stream(stream)))

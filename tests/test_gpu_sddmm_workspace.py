@@ -200,3 +200,31 @@ def test_python_call_on_another_stream_and_captured(dev, orc):
         # two orders of a 64-term dot product
         scale = val.abs() * 64 * lhs.abs().max() * rhs.abs().max()
         assert bool((err <= 1e-5 * scale).all())
+
+
+@pytest.mark.parametrize("rows,asks", [(1000, False), (40000, True)])
+def test_small_calls_do_not_ask_for_scratch(dev, monkeypatch, rows, asks):
+    """The question costs a call of its own; its answer for small calls is
+    0."""
+    csr = _csr(rows, 3001, 5)
+    ro, col, val = G.t(csr.row_offsets), G.t(csr.column_indices), G.t(
+        csr.values)
+    lhs = torch.zeros((csr.rows, 62), device=G.DEV)
+    rhs = torch.zeros((62, csr.cols), device=G.DEV)
+    lib = sw.load_library()
+    asked = []
+
+    class Counting:
+        def __getattr__(self, name):
+            if name == "sw_sddmm_workspace_bytes":
+                asked.append(name)
+            return getattr(lib, name)
+
+    need = lib.sw_sddmm_workspace_bytes(csr.rows, csr.cols, csr.nnz, 62, 4,
+                                        None)
+    assert (need > 0) == asks
+    monkeypatch.setattr(sw, "load_library", lambda: Counting())
+    G.say(f"sddmm asks for scratch, rows={rows}")
+    sw.sddmm(ro, col, val, lhs, rhs, torch.empty_like(val))
+    torch.cuda.synchronize()
+    assert bool(asked) == asks
