@@ -2511,12 +2511,16 @@ bool few_products(int64_t nnz, int64_t kdim) { return nnz < 8000000 / kdim; }
 // thread per row / wave / transposed: 10,000 rows of 8, kdim = 16 29.7 / 10.5 /
 // 14.1; 30,000 of 8, kdim = 4 11.1 / 9.1 / 14.1; 60,000 of 8, kdim = 16 56 /
 // 48 / 19.5).  A wave per row costs with the rows, whatever they hold, a
-// thread per row with the longest row: 1,000,000 rows of one, kdim = 4 88 /
-// 302 / 28; 60,000 of 3, kdim = 8 13 / 23 / 14.
+// thread per row with the longest row, and from kdim = 16 on with the lines
+// of rhs that its lanes gather at once: 1,000,000 rows of one, kdim = 4 88 /
+// 302 / 28; 60,000 of 3, kdim = 8 13 / 23 / 14; 100,000 of one, kdim = 16 86 /
+// 78, bf16 92 / 59; 400,000 of 0.2, kdim = 16 55 / 102, of 0.01, kdim = 64 (in
+// 1,000,000 rows) 210 / 111.
 bool small_sddmm(int64_t rows, int64_t nnz, int64_t kdim) {
   return few_products(nnz, kdim) &&
          (rows <= 16384 || (rows <= 32768 && nnz / 8 >= rows) ||
-          (rows <= 65536 && kdim >= 16));
+          (kdim >= 16 &&
+           (rows <= 65536 || nnz >= rows || nnz < rows / 64)));
 }
 
 // Bytes of scratch memory with which launch_sddmm transposes rhs first (0:
