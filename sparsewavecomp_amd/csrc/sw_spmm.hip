@@ -29,8 +29,9 @@ namespace {
 // Rows of more than kLongSteps steps are taken by the whole wave, one after
 // another (G < 64).  A row's sum has a fixed order.  Units run in XCD chunks:
 // with a contiguous eighth of the rows per XCD, rows sorted by length (200,000
-// of 20 on average, lognormal with sigma 1.5, k = 100, fp32) took 1076 us,
-// 467 so, one thread per output 439; unsorted rows are within 2% either way.
+// of 20 on average, lognormal with sigma 1.5, k = 100, fp32) took 1076 us, 460
+// so, one thread per output 439; unsorted rows within 1%.  (Chunks from both
+// ends of the rows in turn: 373 us sorted, unsorted 1% slower.)
 // Bound by the gathered rows' trips from L2 and the MALL: 200,003 rows of 20
 // entries on average, k = 100, bf16: 268 us one thread per output, 187 us
 // here (0.8 GB of rhs rows).  The mapping thread-per-output: the reference's
