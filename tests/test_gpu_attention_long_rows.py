@@ -139,9 +139,10 @@ def test_long_rows_non_finite_value(dev, orc):
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 def test_defaults_with_shared_buffers(dev, dt):
-    """Without options, a score buffer that is the mask buffer or an output
-    that is the query buffer gives what separate buffers give: such calls
-    keep the six kernels.  (Compared within the chain's rounding: the six
+    """Without options, a score buffer that is the mask buffer, an output that
+    is the query buffer, and an output that is the key buffer (which one
+    kernel would overwrite under tiles still reading it) give what separate
+    buffers give: such calls keep the six kernels.  (Compared within the chain's rounding: the six
     kernels sum in another order than the fused one.)"""
     mask = W.attention_mask(seq=512, block=64, window=3, random_blocks=1,
                             seed=1)
@@ -151,10 +152,10 @@ def test_defaults_with_shared_buffers(dev, dt):
     mv, q, kt, v = (rnd(mask.nnz), rnd(512, 64), rnd(64, 512), rnd(512, 64))
     new = lambda *s: torch.full(s, float("nan"), device=G.DEV, dtype=dt)
 
-    def run(mask_values, query, scores, out):
+    def run(mask_values, query, scores, out, keys=kt):
         rmax, rsum = new(512), new(512)
-        sw.sparse_attention(ro, col, mask_values, query, kt, v, scores, rmax,
-                            rsum, out, 0.125, 1.0)
+        sw.sparse_attention(ro, col, mask_values, query, keys, v, scores,
+                            rmax, rsum, out, 0.125, 1.0)
         torch.cuda.synchronize()
         return [t.double() for t in (scores, rmax, rsum, out)]
 
@@ -165,7 +166,9 @@ def test_defaults_with_shared_buffers(dev, dt):
     # fp32: a few rounding errors of sums of up to 256 terms; bf16: the
     # scores' rounding (2^-9 of scores up to 8) moved by the order
     tol = 2e-5 if dt == torch.float32 else 0.05
+    keys = kt.clone()
     for got in (run(same, q, same, new(512, 64)),
-                run(mv, onto, new(mask.nnz), onto)):
+                run(mv, onto, new(mask.nnz), onto),
+                run(mv, q, new(mask.nnz), keys.view(512, 64), keys)):
         for a, b in zip(got, want):
             assert float((a - b).norm() / b.norm()) <= tol

@@ -112,8 +112,8 @@ def test_bf16_sddmm(dev, orc, golden, opts):
             _sddmm_check(orc, csr, csr.values, lhs, rhs, kind, 0.3, 0.7, got)
 
 
-# the 16-row tiles (row-tile-mfma) and thread-per-row, whose waves take
-# their 64 rows as one matrix-core tile at kdim 64 and 128
+# the 16-row tiles asked for, and calls that choose them for the block mask at
+# kdim 64 and 128 (kdim 256 and the smaller masks: one wave per row)
 TILE_OPTS = ["sddmm-mapping=row-tile-mfma", "", "sddmm-block-size=128"]
 
 

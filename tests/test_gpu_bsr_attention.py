@@ -170,6 +170,9 @@ def test_bsr_config4_sample(dev, orc, opts):
 
 # ---- SDDMM / row reduce / row-wise map / attention -------------------------
 
+# (products as few as in most of these tests take one wave per row whatever
+# the SDDMM block size; test_gpu_sddmm_workspace.py and test_gpu_sddmm_tile64.py
+# run one row per work-item in every block size)
 ROW_OPTS = ["", "sddmm-lanes-per-row=64", "sddmm-block-size=64",
             "sddmm-block-size=512", "sddmm-block-size=1024",
             "sddmm-mapping=row-tile-mfma", "sddmm-mapping=wave-per-row"]
@@ -672,16 +675,15 @@ def _check_attention(orc, csr, scores, rmax, rsum, out, refs, v, inputs):
 
 
 @pytest.mark.parametrize("opts", ["sddmm-mapping=row-tile-mfma",
-                                  # thread-per-row: 64-row wave tiles
                                   "", "sddmm-block-size=128",
                                   "sddmm-block-size=64"])
 @pytest.mark.parametrize("in_place", [False, True])
 @pytest.mark.parametrize("kdim", [64, 128, 32])
 def test_sddmm_tile_mfma_block_mask(dev, orc, kdim, in_place, opts):
-    """Block-structured masks take the 16-row MFMA tiles (row-tile-mfma) or
-    the 64-row wave tiles (thread-per-row, fp32, kdim 64 or 128); with the
-    output in place of the sample values the tiles read each entry's sample
-    before writing it."""
+    """Block masks at kdim 64 and 128 take 16-row matrix-core tiles, asked for
+    or not.  In place the tiles read each entry's sample before writing it
+    when they are asked for; otherwise, and at kdim 32, one wave takes a
+    row."""
     mask = W.attention_mask(seq=2048, block=64, window=4, random_blocks=2,
                             seed=3)
     rng = np.random.default_rng(kdim)

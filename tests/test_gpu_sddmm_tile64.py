@@ -1,8 +1,9 @@
 """The thread-per-row SDDMM's 64-row wave tiles against the CPU oracle.
 
-With the reference's thread-per-row mapping, workgroups of whole waves up to
-256 work-items and kdim 64 or 128, each wave first tries its 64 consecutive
-rows as one matrix-core tile: its structure check reads every column index
+Without scratch memory, a mapping, or rows of 96 entries in the mean, 8 million
+products and more run one row per work-item; in workgroups of whole waves up
+to 256 work-items and with kdim 64 or 128, each wave first tries its 64
+consecutive rows as one matrix-core tile: its structure check reads every column index
 of the tile (16-byte windows, each kept inside the tile's positions) and
 accepts the tile when every row's columns are a prefix of its last row's,
 which holds at most 512 entries and at least 4; other tiles run one row per
@@ -12,7 +13,8 @@ check tells apart:
   rows' own path), leading rows empty or full;
 * prefix tiles with one row's first or last column replaced, or one row
   longer than the last (the check fails);
-* tiles of empty rows and of independent random rows;
+* tiles of empty rows (enough of them to keep the mean row below 96) and of
+  independent random rows;
 and the matrix ends in a prefix tile whose last row holds 4 entries (its
 windows clamped at the arrays' end), 2 entries, or in a partial tile of 37
 rows.  fp32 within the op bar (1e-5 sum |terms|), bf16 within the fp32 bar
@@ -25,7 +27,7 @@ import sparsewavecomp_amd as sw
 from sparsewavecomp_amd import workloads as W
 from tests import gpu_util as G
 from tests._check import assert_within_bound
-from tests.test_gpu_bf16 import _sddmm, _sddmm_check
+from tests.test_gpu_bf16 import _sddmm_check
 
 pytestmark = pytest.mark.gpu
 
@@ -67,7 +69,7 @@ def _tile64_mask(seed, ending):
         else:
             tile[r] = np.array([rng.choice(others)])
         rows_cols += tile
-    rows_cols += [np.zeros(0, np.int64) for _ in range(64)]
+    rows_cols += [np.zeros(0, np.int64) for _ in range(64 * 10)]
     rows_cols += [np.sort(rng.choice(COLS, int(rng.integers(0, 200)),
                                      replace=False)) for _ in range(64)]
     if ending == "last4":
@@ -82,6 +84,28 @@ def _tile64_mask(seed, ending):
     col = np.concatenate(rows_cols).astype(np.int32)
     val = rng.uniform(-1, 1, col.size).astype(np.float32)
     return W.CSR(len(rows_cols), COLS, ro, col, val), rng
+
+
+def _run(csr, lhs, rhs, kind, opts, dt):
+    """The C entry without scratch memory: one row per work-item."""
+    lib = sw.load_library()
+    o = sw.Options.parse(opts) if opts else sw.Options()
+    ro, col = G.t(csr.row_offsets), G.t(csr.column_indices)
+    val, l_, r_ = (G.t(a).to(dt) for a in (csr.values, lhs, rhs))
+    out = torch.full((csr.nnz,), float("nan"), dtype=dt, device=G.DEV)
+    kdim = lhs.shape[1]
+    # rows for which scratch memory would help are neither few nor a block
+    # mask's: without it they are a work-item each
+    assert lib.sw_sddmm_workspace_bytes(csr.rows, csr.cols, csr.nnz, kdim,
+                                        val.element_size(), o.ref) > 0
+    assert csr.nnz * kdim >= 8000000
+    fn = (lib.sw_sddmm_csr_f32 if dt == torch.float32
+          else lib.sw_sddmm_csr_bf16)
+    rc = fn(*(x.data_ptr() for x in (ro, col, val, l_, r_, out)), csr.rows,
+            csr.cols, csr.nnz, kdim, kind, 0.3, 0.7, o.ref, None)
+    torch.cuda.synchronize()
+    assert rc == 0, lib.sw_last_error()
+    return out.float().cpu().numpy()
 
 
 @pytest.mark.parametrize("ending", ["last4", "last2", "partial"])
@@ -102,12 +126,8 @@ def test_sddmm_wave_tiles_f32(dev, orc, kdim, ending):
         for opts in OPTS:
             G.say(f"sddmm wave tiles {ending} kdim={kdim} kind={kind} "
                   f"opts='{opts}'")
-            out = torch.full((csr.nnz,), float("nan"), device=G.DEV)
-            sw.sddmm(G.t(csr.row_offsets), G.t(csr.column_indices),
-                     G.t(csr.values), G.t(lhs), G.t(rhs), out, kind, 0.3, 0.7,
-                     options=opts or None)
-            torch.cuda.synchronize()
-            assert_within_bound(out.cpu().numpy(), ref, bound + 1e-30,
+            got = _run(csr, lhs, rhs, kind, opts, torch.float32)
+            assert_within_bound(got, ref, bound + 1e-30,
                                 what=f"{ending} kind {kind} {opts}")
 
 
@@ -119,6 +139,7 @@ def test_sddmm_wave_tiles_bf16(dev, orc, kdim, ending):
     rhs = rng.standard_normal((kdim, csr.cols)).astype(np.float32)
     for kind in (sw.SDDMM_MUL, sw.SDDMM_AFFINE, sw.SDDMM_DOT):
         for opts in OPTS:
-            got = _sddmm(csr, csr.values, lhs, rhs, kind, 0.3, 0.7,
-                         opts or None)
+            G.say(f"sddmm wave tiles bf16 {ending} kdim={kdim} kind={kind} "
+                  f"opts='{opts}'")
+            got = _run(csr, lhs, rhs, kind, opts, torch.bfloat16)
             _sddmm_check(orc, csr, csr.values, lhs, rhs, kind, 0.3, 0.7, got)

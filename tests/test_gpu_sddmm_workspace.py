@@ -107,13 +107,15 @@ def test_kinds_and_alignment(dev, orc, kind, offset, in_place, dt):
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("opts", [None, "sddmm-block-size=64",
+                                  "sddmm-block-size=512",
+                                  "sddmm-block-size=1024",
                                   "sddmm-mapping=wave-per-row",
                                   "sddmm-mapping=row-tile-mfma"])
 @pytest.mark.parametrize("kdim", [64, 96])
 @pytest.mark.parametrize("rows", [700, 40000])
 def test_without_workspace(dev, orc, rows, kdim, opts, dt):
     """No scratch memory: small calls one wave per row, larger ones by their
-    mapping."""
+    mapping (one row per work-item in workgroups of the block size)."""
     csr = _csr(rows, 3001, 4)
     got, _, ops = _run(csr, kdim, dt, sw.SDDMM_AFFINE, workspace=False,
                        opts=opts)
