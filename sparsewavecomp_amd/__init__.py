@@ -315,10 +315,18 @@ def _workspace(nbytes, like, stream):
     if (like.device.index != torch.cuda.current_device()
             or torch.cuda.is_current_stream_capturing()):
         return None
+    # A new allocation from the driver would invalidate a graph capture that
+    # another thread has under way, unless this thread's interaction mode is
+    # relaxed (2); nothing of this call belongs to that capture.
+    exchange = load_library().hipThreadExchangeStreamCaptureMode
+    mode = ctypes.c_int(2)
+    exchange(ctypes.byref(mode))
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
     except torch.cuda.OutOfMemoryError:
         return None
+    finally:
+        exchange(ctypes.byref(mode))
 
 
 def spmv(row_offsets, column_indices, values, vector, output, options=None,

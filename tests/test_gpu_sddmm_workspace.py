@@ -7,6 +7,7 @@ one of thousands of entries, more than 64 rows to a wave, in place, aligned
 and element-aligned operands, with and without samples.  Bar: the SDDMM's
 1e-5 (|sample| sum |lhs rhs|), plus one rounding in bf16."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -230,3 +231,43 @@ def test_small_calls_do_not_ask_for_scratch(dev, monkeypatch, rows, asks):
     sw.sddmm(ro, col, val, lhs, rhs, torch.empty_like(val))
     torch.cuda.synchronize()
     assert bool(asked) == asks
+
+
+def test_scratch_while_another_thread_captures(dev):
+    """A call on one thread's stream takes its scratch memory also when the
+    allocator has to ask the driver for it while another thread captures a
+    graph, and leaves that capture alone."""
+    csr = _csr(40000, 3001, 7)
+    g = torch.Generator(device=G.DEV).manual_seed(1)
+    lhs = torch.randn((csr.rows, 64), generator=g, device=G.DEV)
+    rhs = torch.randn((64, csr.cols), generator=g, device=G.DEV)
+    ro, col, val = G.t(csr.row_offsets), G.t(csr.column_indices), G.t(
+        csr.values)
+    want = sw.sddmm(ro, col, val, lhs, rhs, torch.empty_like(val))
+    out = torch.empty_like(val)
+    a, b = torch.ones(1000, device=G.DEV), torch.empty(1000, device=G.DEV)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()  # the next scratch memory is a new allocation
+    failed = []
+
+    def other():
+        try:
+            with torch.cuda.stream(side):
+                sw.sddmm(ro, col, val, lhs, rhs, out)
+        except Exception as e:  # noqa: BLE001 (reported below)
+            failed.append(e)
+
+    G.say("sddmm while another thread captures")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        torch.mul(a, 3.0, out=b)
+        thread = threading.Thread(target=other)
+        thread.start()
+        thread.join(30)
+    assert not thread.is_alive() and not failed, failed
+    b.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(b, torch.full_like(b, 3.0))
+    assert torch.equal(out, want)

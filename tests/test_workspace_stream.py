@@ -2,6 +2,7 @@
 devices, which no test machine here has): the memory is taken on the stream
 that the kernel runs on, or not at all."""
 import contextlib
+import ctypes
 import types
 
 import pytest
@@ -16,7 +17,7 @@ class _Stream:
 
 def _fake_torch(capturing=False):
     state = types.SimpleNamespace(device=0, streams={0: "s0", 1: "s1"},
-                                  taken=[])
+                                  taken=[], mode=0)
 
     @contextlib.contextmanager
     def stream(s):
@@ -29,7 +30,9 @@ def _fake_torch(capturing=False):
 
     def empty(nbytes, dtype, device):
         # torch's allocator: the memory belongs to the current stream of the
-        # device that it lies on
+        # device that it lies on; taken in relaxed mode, so that another
+        # thread's capture is left alone
+        assert state.mode == 2
         state.taken.append((device.index, state.streams[device.index]))
         return "memory"
 
@@ -39,6 +42,18 @@ def _fake_torch(capturing=False):
         is_current_stream_capturing=lambda: capturing,
         OutOfMemoryError=MemoryError)
     return types.SimpleNamespace(cuda=cuda, uint8="u8", empty=empty), state
+
+
+def _use(monkeypatch, torch, state):
+    """The stand-in in torch's place, and one for the capture mode."""
+    def exchange(ref):
+        mode = ctypes.cast(ref, ctypes.POINTER(ctypes.c_int))
+        state.mode, mode[0] = mode[0], state.mode
+        return 0
+
+    monkeypatch.setattr(sw, "_torch", torch)
+    monkeypatch.setattr(sw, "load_library", lambda: types.SimpleNamespace(
+        hipThreadExchangeStreamCaptureMode=exchange))
 
 
 def _like(index):
@@ -53,7 +68,7 @@ def _like(index):
 ])
 def test_scratch_lies_on_the_launch_stream(monkeypatch, operands, side, want):
     torch, state = _fake_torch()
-    monkeypatch.setattr(sw, "_torch", torch)
+    _use(monkeypatch, torch, state)
     stream = None if side is None else _Stream(side)
     got = sw._workspace(64, _like(operands), stream)
     if want is None:
@@ -62,11 +77,12 @@ def test_scratch_lies_on_the_launch_stream(monkeypatch, operands, side, want):
         assert got == "memory"
         device, on = state.taken[0]
         assert (device, "side" if on is stream else on) == want
+    assert state.mode == 0
 
 
 def test_no_scratch_under_capture_or_on_a_raw_stream(monkeypatch):
     torch, state = _fake_torch(capturing=True)
-    monkeypatch.setattr(sw, "_torch", torch)
+    _use(monkeypatch, torch, state)
     assert sw._workspace(64, _like(0), None) is None
     assert sw._workspace(64, _like(0), object()) is None
     assert state.taken == []
