@@ -249,25 +249,15 @@ __device__ __forceinline__ void st4_nt(uint16_t *p, v4f v) {
   __builtin_nontemporal_store(v2u{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)},
                               reinterpret_cast<v2u *>(p));
 }
-// The same at element alignment (one 16- or 8-byte access: gfx9-family GPUs
-// under ROCm run with unaligned global access enabled).
+// The same at element alignment (one 16-byte access: gfx9-family GPUs under
+// ROCm run with unaligned global access enabled).
 __device__ __forceinline__ v4f ld4_any(const float *p) {
   v4f v;
   __builtin_memcpy(&v, p, sizeof v);
   return v;
 }
-__device__ __forceinline__ v4f ld4_any(const uint16_t *p) {
-  v2u w;
-  __builtin_memcpy(&w, p, sizeof w);
-  return v4f{bf16_to_f32(w.x & 0xFFFFu), bf16_to_f32(w.x >> 16),
-             bf16_to_f32(w.y & 0xFFFFu), bf16_to_f32(w.y >> 16)};
-}
 __device__ __forceinline__ void st4_any(float *p, v4f v) {
   __builtin_memcpy(p, &v, sizeof v);
-}
-__device__ __forceinline__ void st4_any(uint16_t *p, v4f v) {
-  const v2u w = v2u{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
-  __builtin_memcpy(p, &w, sizeof w);
 }
 template <typename T>
 __device__ __forceinline__ void st1_nt(T *p, float v) {
