@@ -1069,56 +1069,42 @@ __device__ __forceinline__ void attention_long_tile(
   };
   // A.  The next columns a step ahead (two chunks' gathers in flight
   // measured no faster).
-  constexpr int CA = 1;
   float m = -INFINITY;
-  uint32_t cn[CA];
-#pragma unroll
-  for (int h = 0; h < CA; ++h)
-    cn[h] = column(16 * (wave + W * h));
-  for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W * CA) {
-    Op a[CA][S];
-    Win mw[CA];
-#pragma unroll
-    for (int h = 0; h < CA; ++h) {
-      gather_k(cn[h], a[h]);
-      mw[h] = Win{};
-      if constexpr (!NS)
-        mw[h] = window(mask, t0 + 16 * W * h);
-    }
-#pragma unroll
-    for (int h = 0; h < CA; ++h)
-      cn[h] = column(t0 + 16 * W * (CA + h));
+  uint32_t cn = column(16 * wave);
+  for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W) {
+    Op a[S];
+    gather_k(cn, a);
+    Win mw = Win{};
+    if constexpr (!NS)
+      mw = window(mask, t0);
+    cn = column(t0 + 16 * W);
     __builtin_amdgcn_sched_barrier(0);
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kF32) {
+      v4f acc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < CA; ++h) {
-      const int32_t th = t0 + 16 * W * h;
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (kF32) {
-        v4f acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int st = 0; st < S; st += 2) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][st], qb[st], acc,
-                                                     0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              a[h][st + 1], qb[st + 1], acc1, 0, 0, 0);
-        }
-        acc += acc1;
-      } else {
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-          acc = mfma_16x16x32_bf16(a[h][s], qb[s], acc);
+      for (int st = 0; st < S; st += 2) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], qb[st], acc, 0, 0,
+                                                   0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st + 1], qb[st + 1],
+                                                    acc1, 0, 0, 0);
       }
-      float x[4], sv[4];
-      entries(mw[h], th, x);
+      acc += acc1;
+    } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        sv[v] = as_stored<T>(combine_sddmm(
-            region, valid(th, v) ? x[v] : 0.0f, acc[v], alpha, beta));
-        if constexpr (!SO)
-          m = valid(th, v) ? maximumf(m, sv[v]) : m;
-      }
-      store(th, sv);
+      for (int s = 0; s < S; ++s)
+        acc = mfma_16x16x32_bf16(a[s], qb[s], acc);
     }
+    float x[4], sv[4];
+    entries(mw, t0, x);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      sv[v] = as_stored<T>(combine_sddmm(
+          region, valid(t0, v) ? x[v] : 0.0f, acc[v], alpha, beta));
+      if constexpr (!SO)
+        m = valid(t0, v) ? maximumf(m, sv[v]) : m;
+    }
+    store(t0, sv);
   }
   if constexpr (SO)
     return;
@@ -1175,7 +1161,7 @@ __device__ __forceinline__ void attention_long_tile(
   }
   // C.  The next columns a step ahead; bf16 takes two 64-column blocks of
   // the output in one pass over the entries.
-  constexpr int NB = kF32 ? 1 : 2, CC = 1;
+  constexpr int NB = kF32 ? 1 : 2;
   bool nonfinite = false;
   for (int64_t nb0 = 0; nb0 < dv; nb0 += 64 * NB) {
     const int ntiles0 = (int)std::min<int64_t>(4, (dv - nb0) / 16);
@@ -1186,131 +1172,119 @@ __device__ __forceinline__ void attention_long_tile(
 #pragma unroll
       for (int n = 0; n < 4; ++n)
         acc[j][n] = v4f{0.f, 0.f, 0.f, 0.f};
-    uint32_t cc[CC];
+    uint32_t cc = column(16 * wave);
+    for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W) {
+      Win bq[NB][4];
+      const Win y = window(scores, t0);
 #pragma unroll
-    for (int h = 0; h < CC; ++h)
-      cc[h] = column(16 * (wave + W * h));
-    for (int32_t t0 = 16 * wave; t0 < len_last; t0 += 16 * W * CC) {
-      Win y[CC], bq[CC][NB][4];
+      for (int st = 0; st < 4; ++st) {
+        const uint32_t cs = (uint32_t)__builtin_amdgcn_ds_bpermute(
+            (4 * g + st) << 2, (int)cc);
+        if constexpr (IL || !kF32) {
+          const uint32_t vo =
+              (uint32_t)sizeof(T) * (cs * (uint32_t)dv + 4u * (uint32_t)i);
+          bq[0][st] =
+              *reinterpret_cast<const Win *>(at_bytes(value + nb0, vo));
+          if constexpr (NB == 2) {
+            bq[1][st] = Win{};
+            if (both)
+              bq[1][st] = *reinterpret_cast<const Win *>(
+                  at_bytes(value + nb0 + 64, vo));
+          }
+        } else {
+          const uint32_t vo = 4u * (cs * (uint32_t)dv + (uint32_t)i);
 #pragma unroll
-      for (int h = 0; h < CC; ++h) {
-        y[h] = window(scores, t0 + 16 * W * h);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const uint32_t cs = (uint32_t)__builtin_amdgcn_ds_bpermute(
-              (4 * g + st) << 2, (int)cc[h]);
-          if constexpr (IL || !kF32) {
-            const uint32_t vo = (uint32_t)sizeof(T) *
-                                (cs * (uint32_t)dv + 4u * (uint32_t)i);
-            bq[h][0][st] =
-                *reinterpret_cast<const Win *>(at_bytes(value + nb0, vo));
-            if constexpr (NB == 2) {
-              bq[h][1][st] = Win{};
-              if (both)
-                bq[h][1][st] = *reinterpret_cast<const Win *>(
-                    at_bytes(value + nb0 + 64, vo));
-            }
-          } else {
-            const uint32_t vo = 4u * (cs * (uint32_t)dv + (uint32_t)i);
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-              const int nn = n < ntiles0 ? n : 0; // wave-uniform
-              bq[h][0][st][n] = *at_bytes(value + nb0 + 16 * nn, vo);
-            }
+          for (int n = 0; n < 4; ++n) {
+            const int nn = n < ntiles0 ? n : 0; // wave-uniform
+            bq[0][st][n] = *at_bytes(value + nb0 + 16 * nn, vo);
           }
         }
       }
-#pragma unroll
-      for (int h = 0; h < CC; ++h)
-        cc[h] = column(t0 + 16 * W * (CC + h));
+      cc = column(t0 + 16 * W);
       __builtin_amdgcn_sched_barrier(0);
+      float p[4];
+      if (nb0 == 0) { // P from the scores, stored over them
+        exps(y, t0, p);
 #pragma unroll
-      for (int h = 0; h < CC; ++h) {
-        const int32_t th = t0 + 16 * W * h;
-        float p[4];
-        if (nb0 == 0) { // P from the scores, stored over them
-          exps(y[h], th, p);
+        for (int v = 0; v < 4; ++v) {
+          p[v] = as_stored<T>(tile_div<LIBM>(p[v], sum, rsum_i));
+          p[v] = valid(t0, v) ? p[v] : 0.0f;
+        }
+        store(t0, p);
+      } else { // P as the first pass stored it
+        entries(y, t0, p);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            p[v] = as_stored<T>(tile_div<LIBM>(p[v], sum, rsum_i));
-            p[v] = valid(th, v) ? p[v] : 0.0f;
+        for (int v = 0; v < 4; ++v)
+          p[v] = valid(t0, v) ? p[v] : 0.0f;
+      }
+      if constexpr (kF32) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int st = 0; st < 4; ++st)
+            acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                p[st], bq[0][st][n], acc[0][n], 0, 0, 0);
+      } else {
+        const v2u pk = v2u{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int n = 0; n < 4; ++n) {
+            const v2u bn = v2u{bf16_pair(bq[j][0], bq[j][1], n),
+                               bf16_pair(bq[j][2], bq[j][3], n)};
+            acc[j][n] = mfma_16x16x16_bf16(pk, bn, acc[j][n]);
           }
-          store(th, p);
-        } else { // P as the first pass stored it
-          entries(y[h], th, p);
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            p[v] = valid(th, v) ? p[v] : 0.0f;
-        }
-        if constexpr (kF32) {
-#pragma unroll
-          for (int n = 0; n < 4; ++n)
-#pragma unroll
-            for (int st = 0; st < 4; ++st)
-              acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                  p[st], bq[h][0][st][n], acc[0][n], 0, 0, 0);
-        } else {
-          const v2u pk = v2u{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-              const v2u bn = v2u{bf16_pair(bq[h][j][0], bq[h][j][1], n),
-                                 bf16_pair(bq[h][j][2], bq[h][j][3], n)};
-              acc[j][n] = mfma_16x16x16_bf16(pk, bn, acc[j][n]);
-            }
-        }
       }
     }
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-    const int64_t nb = nb0 + 64 * j;
-    if (nb >= dv)
-      break; // wave-uniform
-    const int ntiles = (int)std::min<int64_t>(4, (dv - nb) / 16);
+      const int64_t nb = nb0 + 64 * j;
+      if (nb >= dv)
+        break; // wave-uniform
+      const int ntiles = (int)std::min<int64_t>(4, (dv - nb) / 16);
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        part[wave][n][v][l] = acc[j][n][v];
-    __syncthreads();
-    if (wave < (IL || !kF32 ? 4 : ntiles)) {
-      // IL: wave w finishes rows 4g + w, columns nb + 4i .. nb + 4i + 3;
-      // else wave n the tile of columns nb + 16n + i, rows 4g + v
-      float o[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        o[x] = 0.0f;
-#pragma unroll
-        for (int w = 0; w < W; ++w)
-          o[x] += IL || !kF32 ? part[w][x][wave][l] : part[w][wave][x][l];
-      }
-      if constexpr (IL || !kF32) {
-        const int rr = 4 * g + wave;
-        if (rr < nt) {
-          T *dst = out + (int64_t)(r0 + rr) * dv + nb + 4 * i;
-          if constexpr (kF32)
-            *reinterpret_cast<v4f *>(dst) = v4f{o[0], o[1], o[2], o[3]};
-          else
-            *reinterpret_cast<v2u *>(dst) =
-                v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-#pragma unroll
-          for (int x = 0; x < 4; ++x)
-            nonfinite |= !__builtin_isfinite(o[x]);
-        }
-      } else {
+      for (int n = 0; n < 4; ++n)
 #pragma unroll
         for (int v = 0; v < 4; ++v)
-          if (4 * g + v < nt) {
-            stv(out + (int64_t)(r0 + 4 * g + v) * dv + nb + 16 * wave + i,
-                o[v]);
-            nonfinite |= !__builtin_isfinite(o[v]);
+          part[wave][n][v][l] = acc[j][n][v];
+      __syncthreads();
+      if (wave < (IL || !kF32 ? 4 : ntiles)) {
+        // IL: wave w finishes rows 4g + w, columns nb + 4i .. nb + 4i + 3;
+        // else wave n the tile of columns nb + 16n + i, rows 4g + v
+        float o[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          o[x] = 0.0f;
+#pragma unroll
+          for (int w = 0; w < W; ++w)
+            o[x] += IL || !kF32 ? part[w][x][wave][l] : part[w][wave][x][l];
+        }
+        if constexpr (IL || !kF32) {
+          const int rr = 4 * g + wave;
+          if (rr < nt) {
+            T *dst = out + (int64_t)(r0 + rr) * dv + nb + 4 * i;
+            if constexpr (kF32)
+              *reinterpret_cast<v4f *>(dst) = v4f{o[0], o[1], o[2], o[3]};
+            else
+              *reinterpret_cast<v2u *>(dst) =
+                  v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              nonfinite |= !__builtin_isfinite(o[x]);
           }
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (4 * g + v < nt) {
+              stv(out + (int64_t)(r0 + 4 * g + v) * dv + nb + 16 * wave + i,
+                  o[v]);
+              nonfinite |= !__builtin_isfinite(o[v]);
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(nonfinite) != 0 && l == 0)
+          v_nonfinite = 1;
       }
-      if (__builtin_amdgcn_ballot_w64(nonfinite) != 0 && l == 0)
-        v_nonfinite = 1;
-    }
-    __syncthreads();
+      __syncthreads();
     }
   }
   // (the barrier above also made every wave's stored P visible)
