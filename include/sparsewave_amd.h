@@ -75,10 +75,16 @@ typedef struct sw_options {
                                        wave-per-row-tile-lds (the last four
                                        are Wave64 extensions; -lds stages the
                                        RHS rows in LDS) */
-  int64_t spmm_block_size;          /* 1..1024, default 256 */
-  int64_t spmm_tile_size;           /* 1..32, default 4 */
+  int64_t spmm_block_size;          /* 1..1024, default 256; thread-per-output
+                                       and the bf16 and wider-than-k row tiles
+                                       choose their own */
+  int64_t spmm_tile_size;           /* 1..32, default 4; bf16 row tiles, and
+                                       tiles wider than k, run the lane groups
+                                       of thread-per-output */
   int64_t spmm_position_chunk_size; /* default 1 */
-  int64_t sddmm_block_size;         /* default 256 */
+  int64_t sddmm_block_size;         /* default 256: the workgroup of SDDMM's
+                                       kernel with one row per work-item; the
+                                       other kernels' are fixed */
   int64_t row_reduction_block_size; /* default 256, rounded up to whole waves */
   int64_t rowwise_map_block_size;   /* default 256 (checked; the maps' blocks
                                        are fixed) */
@@ -94,21 +100,29 @@ typedef struct sw_options {
   int64_t spmm_lanes_per_row;       /* wave-per-row-tile: lanes per (row,
                                        tile) group, power of two, default 64 */
   int64_t bsr_use_mfma;             /* BSR SpMM: 1 = MFMA tiles when the block
-                                       size allows it (default), 0 = the
+                                       size and the products per block row
+                                       are worth it (default), 0 = the
                                        thread-per-output kernel */
   int64_t sddmm_lanes_per_row;      /* SDDMM: 1 = the mapping's own choice
-                                       (default); 64 = one wave per row with
-                                       lanes split over the dot products */
+                                       (default); 64 = one wave per row, as
+                                       sddmm-mapping=wave-per-row */
   int64_t spmm_positions_per_lane;  /* SpMM wave-per-position: consecutive
                                        positions per lane group 1,2,4,8,16;
                                        default 4 */
   char sddmm_mapping[32];           /* thread-per-row (default: the
                                        launch is chosen by size and mean row
-                                       length) | wave-per-row | row-tile-mfma (16-row
-                                       tiles on the matrix cores; tiles whose
-                                       rows do not share column structure,
-                                       and kdim not in {64,128,256}, use the
-                                       vector path) */
+                                       length) | wave-per-row | row-tile-mfma
+                                       (16-row tiles on the matrix cores;
+                                       tiles whose rows do not share column
+                                       structure run one wave per row).  A
+                                       call given scratch memory transposes
+                                       rhs under the first two, and under
+                                       row-tile-mfma with kdim not in
+                                       {64,128,256}, instead of running the
+                                       mapping (see sw_sddmm_workspace_bytes);
+                                       without it wave-per-row, and
+                                       row-tile-mfma at those kdim, are one
+                                       wave per row */
 } sw_options;
 
 /* Fill `opts` with the defaults. */
@@ -272,11 +286,13 @@ int sw_bsr_slab_floor(const int32_t *block_row_offsets,
  * sparsewave.sddmm: output_values[p] = region(values[p], lhs[r,:] . rhs[:,c])
  * for every stored (r, c) at position p.  lhs[rows][kdim], rhs[kdim][cols]
  * row-major.  ThreadPerRowSDDMMPattern (SparseWaveToGPU.cpp:667-750).
- * Rows of more than 96 entries in the mean (kdim 64 or 128) and
- * sddmm-mapping=row-tile-mfma run 16-row v_mfma_f32_16x16x4_f32 tiles for
- * kdim in {64,128,256}; with kdim 64 or 128, at least 4 entries, and
- * output_values not overlapping values (or SW_SDDMM_DOT), the tiles are the
- * fused attention kernel's product phase.  Other kdim take one wave per row.
+ * sddmm-mapping=row-tile-mfma with kdim in {64,128,256}, and rows of more
+ * than 96 entries in the mean with kdim 64 or 128 where no wave per row was
+ * asked for, run 16-row v_mfma_f32_16x16x4_f32 tiles; with kdim 64 or 128, at
+ * least 4 entries, and output_values not overlapping values (or
+ * SW_SDDMM_DOT), the tiles are the fused attention kernel's product phase.
+ * Rows past 96 entries at other kdim, and few products in few rows, take one
+ * wave per row; the rest one work-item per row.
  */
 int sw_sddmm_csr_f32(const int32_t *row_offsets, const int32_t *column_indices,
                      const float *values, const float *lhs, const float *rhs,
@@ -305,7 +321,8 @@ int sw_sddmm_csr_bf16(const int32_t *row_offsets,
  * there first and each entry reads consecutive elements (graphs; block
  * masks run on matrix-core tiles without it).  A null, short or misaligned
  * workspace is ignored.  The workspace belongs to the call until its work
- * on `stream` is done.
+ * on `stream` is done.  The transposition takes the place of wave-per-row
+ * and sddmm-lanes-per-row=64 too; to run those, pass no workspace.
  */
 int64_t sw_sddmm_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz,
                                  int64_t kdim, int value_bytes,
@@ -385,8 +402,9 @@ int sw_csr_rowwise_map_bf16(const int32_t *row_offsets,
  * spmm-mapping=row-tile-mfma, and with every mapping and block size left at
  * its default, one kernel runs the chain over 16-row tiles (d in {64, 128},
  * dv % 16 == 0, nnz >= 4; without options also no output sharing memory
- * with another buffer, the exponentials and divisions then as the separate
- * ops compute them); other calls launch the separate ops.
+ * with another buffer and, past 16,384 rows, eight entries in the mean row,
+ * the exponentials and divisions then as the separate ops compute them);
+ * other calls launch the separate ops.
  */
 int sw_sparse_attention_f32(const int32_t *row_offsets,
                             const int32_t *column_indices,
