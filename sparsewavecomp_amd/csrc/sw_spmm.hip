@@ -940,8 +940,8 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
                                    : 16;
   int G = std::min(64, CL * PL);
   // Few long rows: a wave for each, and narrower tiles of it until there are
-  // a thousand waves (20 rows of 20,000, bf16: k = 128 518 -> 84 us, k = 4
-  // 122 -> 27).
+  // a thousand waves (20 rows of 20,000, bf16: k = 128 518 -> 94 us, k = 4
+  // 122 -> 33).
   auto waves = [&] { return rows * ceil_div(k, (int64_t)CL * V); };
   if (nnz / 48 >= rows && waves() * G / 64 < 2048) {
     G = 64;

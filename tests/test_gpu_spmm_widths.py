@@ -67,6 +67,28 @@ def test_widths(dev, orc, k, mean, opts, offset, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mean", [0.4, 2, 4, 9, 20, 150])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 6, 7, 8, 9, 17, 33, 63, 100, 129])
+def test_entries_at_a_time(dev, orc, k, mean, dt):
+    """Mean rows on every side of the rule that sets how many entries a row's
+    lanes take at a time, with one row past the group's own steps."""
+    rng = np.random.default_rng(k)
+    lens = rng.poisson(mean, 901)
+    lens[450] = max(200, lens[450])
+    csr = W.csr_from_lengths(rng, lens, 1201)
+    rhs = rng.uniform(-1, 1, (csr.cols, k)).astype(np.float32)
+    val = csr.values
+    if dt == torch.bfloat16:
+        val, rhs = G.bf16_round(val), G.bf16_round(rhs)
+    got = _run(csr, val, rhs, dt, None, 0)
+    ref = orc.spmm(csr.row_offsets, csr.column_indices, val, rhs)
+    bound = orc.spmm_abs_bound(csr.row_offsets, csr.column_indices, val, rhs)
+    if dt == torch.bfloat16:
+        bound = bound * (1 + 2.0 ** -8) + 2.0 ** -8 * np.abs(ref) / 1e-5
+    assert_within_bound(got, ref, bound)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("opts", [None, TILE])
 @pytest.mark.parametrize("k", [3, 30, 70])
 def test_inf_reaches_its_rows(dev, orc, k, opts, dt):
