@@ -2505,11 +2505,14 @@ bool small_sddmm(int64_t rows, int64_t nnz, int64_t kdim) {
 // products are worth it from 500,000 elements of lhs on (30,000 rows of 3,
 // kdim = 32 52 us one wave per row, 15.3 transposed; 30,000 of 8, kdim = 4 9.1
 // and 14.1), except the single product of kdim = 1 (1,000,000 rows of 3 41 us
-// one thread per row, 53 transposed).  At most 1 GiB.
+// one thread per row, 53 transposed) and below 200,000 products (100,000 rows
+// of 0.2, kdim = 8 9 and 15, kdim = 16 20 and 15; the allocation and the second
+// launch alone take the host 5).  At most 1 GiB.
 int64_t sddmm_workspace(int64_t rows, int64_t cols, int64_t nnz, int64_t kdim,
                         int64_t elem, const sw_options &o) {
   if (rows <= 0 || cols <= 0 || kdim <= 0 || kdim > INT32_MAX / 2 ||
-      (few_products(nnz, kdim) && (kdim == 1 || rows < 500000 / kdim)) ||
+      (few_products(nnz, kdim) &&
+       (kdim == 1 || rows < 500000 / kdim || nnz < 200000 / kdim)) ||
       nnz < cols / 4 || block_rows(rows, nnz) ||
       (streq(o.sddmm_mapping, "row-tile-mfma") &&
        (kdim == 64 || kdim == 128 || kdim == 256)))

@@ -351,3 +351,22 @@ def test_slab_floor_rejects_shapes_it_does_not_run():
     assert lib.sw_bsr_slab_floor(ok, ok, ok, ok, ok, 30, 32, 2, 8, 4, 4,
                                  None) == -2                  # rows % 16
 
+
+
+def test_sddmm_workspace_rule():
+    """Scratch memory for a transposed rhs is asked for where it pays: not for
+    few products in few rows, nor below 200,000 products in however many
+    rows, block masks, or columns that few entries use."""
+    ask = sw.load_library().sw_sddmm_workspace_bytes
+    graph = (60013, 50021, 960000, 64, 4, None)
+    assert ask(*graph) == 50021 * 64 * 4
+    assert ask(60013, 50021, 960000, 63, 2, None) == 50021 * 64 * 2
+    assert ask(60013, 50021, 960000, 64, 8, None) == 0
+    assert ask(1000, 1000, 10000, 16, 4, None) == 0
+    assert ask(1000000, 50000, 1000000, 4, 4, None) > 0
+    assert ask(1000000, 50000, 3000000, 1, 4, None) == 0
+    assert ask(76760, 149, 3838, 11, 2, None) == 0
+    assert ask(100000, 50000, 20000, 16, 4, None) > 0
+    assert ask(8192, 8192, 2826240, 64, 4, None) == 0
+    assert ask(60013, 50021, 12000, 64, 4, None) == 0
+    assert ask(60013, 1 << 23, 4000000, 64, 4, None) == 0  # past 1 GiB
