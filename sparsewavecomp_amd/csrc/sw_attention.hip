@@ -629,7 +629,7 @@ __global__ __launch_bounds__(1024) void row_reduce_group(
 // Cut by entries: a wave takes N windows of 64 W consecutive positions, W =
 // 16 bytes' worth a lane, so that every load and store is a whole coalesced
 // window whatever the rows' lengths.  The wave finds the rows of its first
-// and last position by scalar searches under the loads, stages the rows'
+// and last position by 64 probes a trip under the loads, stages the rows'
 // ends and values between them in LDS, and each lane searches the row of its
 // first position there and steps on from it; over wider spans each entry
 // searches ro itself.  out may be val (in place): a
@@ -662,9 +662,8 @@ __global__ __launch_bounds__(256) void rowwise_map_positions(
 #pragma unroll
   for (int n = 0; n < N; ++n)
     load_window(val, first + W * (l + kWave * n), nnz, nnz, x[n]);
-  const int fr = row_search_uniform(ro, 1u, (uint32_t)rows, (int32_t)first);
-  const int lr = row_search_gallop(ro, (uint32_t)fr + 1u, (uint32_t)rows,
-                                   (int32_t)last);
+  int fr, lr;
+  row_search_wave(ro, 1, rows, (int32_t)first, (int32_t)last, &fr, &lr);
   const int span = lr - fr; // wave-uniform
   const bool staged = span < kMapRows;
   int32_t *win = ends[wave];

@@ -379,6 +379,48 @@ __device__ __forceinline__ int row_search_gallop(const int32_t *__restrict__ ro,
   return row_search_uniform(ro, lo, hi, pos);
 }
 
+// Two wave-uniform searches over the same range by the whole wave, 64 probes
+// of each a trip: three or four trips for a million rows, where a bisection's
+// twenty dependent probes are not under anything else.  (Vector loads: not for
+// waves whose gathers saturate vector memory.)
+__device__ __forceinline__ void row_search_wave(const int32_t *__restrict__ ro,
+                                                int32_t lo, int32_t hi,
+                                                int32_t pos_a, int32_t pos_b,
+                                                int *row_a, int *row_b) {
+  const int l = lane_id();
+  int32_t from[2] = {lo, lo}, to[2] = {hi, hi};
+  const int32_t pos[2] = {pos_a, pos_b};
+  while (from[0] < to[0] || from[1] < to[1]) { // wave-uniform
+    int32_t v[2];
+    bool in[2];
+    int32_t step[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int32_t n = to[s] - from[s];
+      step[s] = n / kWave + (n % kWave != 0); // (n may be near 2^31)
+      const int64_t at = (int64_t)l * step[s];
+      in[s] = at < n;
+      // (lanes past the range, and a search that is done, probe `lo`)
+      v[s] = ro[in[s] ? from[s] + (int32_t)at : lo];
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const uint64_t live = ballot(in[s]);
+      if (live == 0)
+        continue; // done
+      const uint64_t past = ballot(in[s] && v[s] > pos[s]);
+      // probes 0 .. f - 1 are at or below pos, probe f (if any) past it
+      const int f = past != 0 ? __builtin_ctzll(past) : __builtin_popcountll(live);
+      if (past != 0)
+        to[s] = from[s] + f * step[s];
+      if (f > 0)
+        from[s] += (f - 1) * step[s] + 1;
+    }
+  }
+  *row_a = from[0] - 1;
+  *row_b = from[1] - 1;
+}
+
 // ---- 16-row tiles with shared column structure ------------------------------
 // Rows r0 .. r0+nt-1 (nt <= 16) form an MFMA tile when every row's column
 // list is a prefix of the tile's last row's list -- true for block masks and

@@ -375,3 +375,25 @@ def test_coo_of_one_entry_a_row(dev):
     assert torch.equal(sums[:n], val[:n] * x[col[:n].long()])
     print(f"aligned {even:.1f} us, off by one {odd:.1f} us")
     assert even <= 1.25 * odd
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_row_map_finds_its_rows(dev, dt):
+    """A map over rows of which one in ten holds an entry takes a few more
+    trips than the same entries in a few rows, whose search is short."""
+    rows = 200000
+    lens = (torch.arange(rows) % 10 == 0).long()
+    n = int(lens.sum())
+    few = torch.full((n // 1000,), 1000)
+
+    def call(lens):
+        ro = offsets(lens)
+        val = torch.rand(int(ro[-1]), device=G.DEV).to(dt)
+        rv = torch.rand(lens.numel(), device=G.DEV).to(dt)
+        out = torch.empty_like(val)
+        return lambda: sw.csr_rowwise_map(ro, None, val, rv, out, sw.MAP_SUB)
+
+    G.say(f"row map of {rows} rows {dt}")
+    many, short = us(call(lens)), us(call(few))
+    print(f"many rows {many:.1f} us, few {short:.1f} us")
+    assert many <= 2.5 * short
