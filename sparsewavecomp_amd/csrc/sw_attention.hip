@@ -586,7 +586,26 @@ __global__ __launch_bounds__(1024) void row_reduce_group(
   const int gl = threadIdx.x & (G - 1);
   const bool in = r < rows;
   const int32_t s = in ? ro[r] : 0, e = in ? ro[r + 1] : 0;
-  const bool wide = e - s > kGroupSteps * kRowEntries * G;
+  bool wide = e - s > kGroupSteps * kRowEntries * G;
+  uint64_t m = ballot(wide && gl == 0);
+  if (m != 0) {
+    // the wave's long rows one after another, a trip and more each, unless the
+    // groups' steps over the longest are fewer (neighbours as long, as where
+    // rows are sorted by length: 445,278 rows of 19, bf16, 22.5 us otherwise,
+    // one thread per row 11.9)
+    int32_t longest = 0, trips = 0;
+    for (uint64_t left = m; left != 0; left &= left - 1) { // wave-uniform
+      const int src = __builtin_ctzll(left);
+      const int32_t len = __builtin_amdgcn_readlane(e, src) -
+                          __builtin_amdgcn_readlane(s, src);
+      longest = len > longest ? len : longest;
+      trips += 1 + len / (4 * W * kWave);
+    }
+    if (trips >= longest / (kRowEntries * G)) {
+      wide = false;
+      m = 0;
+    }
+  }
   const int32_t end = wide ? s : e;
   float acc = MAX ? -INFINITY : 0.0f;
   for (int32_t at = s; ballot(at < end) != 0; at += kRowEntries * G) {
@@ -602,7 +621,6 @@ __global__ __launch_bounds__(1024) void row_reduce_group(
   if (in && !wide && gl == 0)
     stv(out + r, acc);
   // the wave's long rows
-  uint64_t m = ballot(wide && gl == 0);
   while (m != 0) { // wave-uniform
     const int src = __builtin_ctzll(m);
     m &= m - 1;

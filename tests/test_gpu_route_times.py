@@ -378,6 +378,25 @@ def test_coo_of_one_entry_a_row(dev):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_row_reduction_of_rows_sorted_by_length(dev, dt):
+    """A wave whose rows are all long reads them side by side."""
+    g = torch.Generator().manual_seed(3)
+    lens = torch.exp(0.7 * torch.randn(450000, generator=g) + 2.7)
+    lens = lens.round().clamp(1, 4096).long()
+
+    def call(lens):
+        ro = offsets(lens)
+        val = torch.rand(int(ro[-1]), device=G.DEV).to(dt)
+        out = torch.empty(lens.numel(), device=G.DEV, dtype=dt)
+        return lambda: sw.csr_row_reduce(ro, None, val, out, "max")
+
+    G.say(f"row reduction of sorted rows {dt}")
+    mixed, up = us(call(lens)), us(call(lens.sort().values))
+    print(f"sorted {up:.1f} us, shuffled {mixed:.1f} us")
+    assert up <= 1.5 * mixed
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 def test_row_map_finds_its_rows(dev, dt):
     """A map over rows of which one in ten holds an entry takes a few more
     trips than the same entries in a few rows, whose search is short."""
