@@ -920,11 +920,14 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
   // rows of rhs at once (fp32, 100,000 rows of 60, k = 128, CL 8 / 16 / 32:
   // 464 / 531 / 618 us, k = 33 221 / 274; 200,003 rows of 20, k = 100 302 /
   // 288 / 320).
-  // From a mean of 128 on whole rows again (5,000 rows of 300, k = 100, CL 8 /
-  // 16: fp32 98 / 90, bf16 53 / 35 us).
+  // From a mean of 128 on whole rows again where they are enough waves (5,000
+  // rows of 300, k = 100, CL 8 / 16: fp32 98 / 90, bf16 53 / 35 us; 522 of 369,
+  // k = 153, fp32 17 / 24; 1,142 of 1,256, k = 209, bf16 182 / 249).
   int V = k >= 8 && sizeof(T) == 2 ? 8 : k >= 4 ? 4 : k >= 2 ? 2 : 1;
-  int CL = next_pow2((int)std::min<int64_t>(
-      ceil_div(k, V), nnz / 48 >= rows && nnz / 128 < rows ? 8 : 16));
+  const bool wide_row =
+      nnz / 48 < rows ||
+      (nnz / 128 >= rows && rows * ceil_div(k, (int64_t)16 * V) >= 4608);
+  int CL = next_pow2((int)std::min<int64_t>(ceil_div(k, V), wide_row ? 16 : 8));
   // PL entries at a time, by the mean row: lanes past a row's entries still
   // take part in its steps and its butterfly.  us, fp32, PL 1 / 2 / 4:
   // 1,000,000 rows of 0.05 entries k = 64 60 / 81 / 132, of 2 108 / 141 / 258,
@@ -941,9 +944,9 @@ int launch_row_group(const int32_t *ro, const int32_t *col, const T *val,
   int G = std::min(64, CL * PL);
   // Few long rows: a wave for each, and narrower tiles of it until there are
   // a thousand waves (20 rows of 20,000, bf16: k = 128 518 -> 94 us, k = 4
-  // 122 -> 33).
+  // 122 -> 33; 10,946 of 35 sorted by length, k = 14 54 -> 20).
   auto waves = [&] { return rows * ceil_div(k, (int64_t)CL * V); };
-  if (nnz / 48 >= rows && waves() * G / 64 < 2048) {
+  if (nnz / 16 >= rows && waves() * G / 64 < 2048) {
     G = 64;
     while (CL > 1 && waves() < 1024)
       CL /= 2;

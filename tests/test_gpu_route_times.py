@@ -416,3 +416,16 @@ def test_row_map_finds_its_rows(dev, dt):
     many, short = us(call(lens)), us(call(few))
     print(f"many rows {many:.1f} us, few {short:.1f} us")
     assert many <= 2.5 * short
+
+
+def test_spmm_of_few_sorted_rows(dev):
+    """A few thousand rows of unequal length are a wave each, so that the
+    longest, side by side, are not one wave's."""
+    g = torch.Generator().manual_seed(3)
+    lens = torch.exp(1.5 * torch.randn(11000, generator=g) + 2.45)
+    lens = lens.round().clamp(1, 4096).long()
+    G.say("spmm of few sorted rows")
+    mixed = us(_spmm_call(lens, 14, torch.bfloat16, cols=20000))
+    up = us(_spmm_call(lens.sort().values, 14, torch.bfloat16, cols=20000))
+    print(f"ascending {up:.1f} us, shuffled {mixed:.1f} us")
+    assert up <= 1.6 * mixed
