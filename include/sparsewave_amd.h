@@ -402,7 +402,7 @@ int sw_csr_rowwise_map_bf16(const int32_t *row_offsets,
  * spmm-mapping=row-tile-mfma, and with every mapping and block size left at
  * its default, one kernel runs the chain over 16-row tiles (d in {64, 128},
  * dv % 16 == 0, nnz >= 4; without options also no output sharing memory
- * with another buffer and, past 16,384 rows, eight entries in the mean row,
+ * with another buffer and, past 16,384 rows, five entries in the mean row,
  * the exponentials and divisions then as the separate ops compute them);
  * other calls launch the separate ops.
  */

@@ -3174,13 +3174,14 @@ int attention_entry(const int32_t *row_offsets, const int32_t *column_indices,
   // memory with another operand (the six kernels finish reading an operand
   // before a later one writes).  3,001 positions of up to 384 entries,
   // d = dv = 64, fp32: 536 us in six kernels, 12.4 us in one.  Not many rows
-  // of fewer than eight entries: tiles of them seldom share columns, and row
+  // of fewer than five entries: tiles of them seldom share columns, and row
   // by row a wave's chain of trips costs the same however short the row is
   // (d = 64, fp32, one kernel / six: 100,000 rows of 0.1 entries 251 / 85 us, of
   // 4 691 / 474, 32,000 in 8 x 8 blocks 156 / 56; 8,000 rows of 4 30 / 46,
-  // 32,000 in 16 x 16 blocks, 8.5 entries a row, 31 / 61).
+  // 32,000 of 8 223 / 196, in 16 x 16 blocks, 8.5 entries a row, 31 / 61; bf16
+  // 23,585 rows of 7.6, unequal and sorted by length, 147 / 336).
   const bool defaults =
-      (rows <= 16384 || nnz / 8 >= rows) &&
+      (rows <= 16384 || nnz / 5 >= rows) &&
       streq(o.sddmm_mapping, "thread-per-row") &&
       streq(o.spmm_mapping, "thread-per-output") &&
       o.sddmm_lanes_per_row == 1 && o.sddmm_block_size == 256 &&
