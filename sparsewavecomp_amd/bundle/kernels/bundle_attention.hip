@@ -334,8 +334,10 @@ __device__ __forceinline__ bool output_tile16(
   // row i's first position and length (lanes of rows past nt: length 0)
   const int ic = i < nt ? i : nt - 1;
   const int32_t ra = __builtin_amdgcn_ds_bpermute(ic << 2, my_ro);
-  const int32_t la =
-      i < nt ? __builtin_amdgcn_ds_bpermute((ic + 1) << 2, my_ro) - ra : 0;
+  // (on every lane: a permute reads zero from a lane that is switched off, and
+  // row nt - 1's end is in lane nt)
+  const int32_t rnext = __builtin_amdgcn_ds_bpermute((ic + 1) << 2, my_ro);
+  const int32_t la = i < nt ? rnext - ra : 0;
   // the last row's columns in LDS, slots past its end repeating its final
   // column; then every row but the last against them: lane l compares
   // entries 4l .. 4l + 3 and 256 + 4l .. + 3, read as element-aligned

@@ -239,7 +239,9 @@ def test_fuzz_bsr(dev, orc, seed):
                 assert rel_l2(got, ref) <= BF16_REL_L2
 
 
-@pytest.mark.parametrize("seed", SEEDS)
+# (seed 30 too: 43 rows, whose last 16-row tile holds 11 rows and is a prefix
+# tile; its last row's length was read from a lane that was switched off)
+@pytest.mark.parametrize("seed", sorted({*SEEDS, 30}))
 def test_fuzz_attention_bundle(dev, orc, tmp_path, seed):
     """The lrrt attention bundle built for each fuzz mask's shapes (its
     kernels specialise rows, key rows, d and dv), its six kernels launched in
