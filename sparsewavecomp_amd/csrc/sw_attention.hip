@@ -2741,11 +2741,13 @@ int launch_sddmm(const int32_t *ro, const int32_t *col, const T *val,
   return launch_check("SDDMM kernel");
 }
 
-// Lanes per row of the row reductions: a mean row in one step.
+// Lanes per row of the row reductions: a mean row in one step, and more of
+// them while the rows are fewer than 2,048 waves (8,548 rows of 11, lognormal
+// with sigma 1.5 and sorted by length, bf16: 2 lanes 31 us, 16 lanes 8).
 int row_lanes(int64_t rows, int64_t nnz) {
   const int64_t mean = nnz / std::max<int64_t>(rows, 1);
   int g = 2;
-  while (g < 64 && kRowEntries * g < mean)
+  while (g < 64 && (kRowEntries * g < mean || rows * g / kWave < 2048))
     g *= 2;
   return g;
 }

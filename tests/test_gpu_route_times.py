@@ -385,10 +385,13 @@ def test_coo_of_one_entry_a_row(dev):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-def test_row_reduction_of_rows_sorted_by_length(dev, dt):
-    """A wave whose rows are all long reads them side by side."""
+@pytest.mark.parametrize("rows,sigma", [(450000, 0.7), (8500, 1.5)])
+def test_row_reduction_of_rows_sorted_by_length(dev, rows, sigma, dt):
+    """A wave whose rows are all long reads them side by side, and few rows
+    are spread over the chip."""
     g = torch.Generator().manual_seed(3)
-    lens = torch.exp(0.7 * torch.randn(450000, generator=g) + 2.7)
+    lens = torch.exp(sigma * torch.randn(rows, generator=g) + 2.7
+                     - (sigma - 0.7))
     lens = lens.round().clamp(1, 4096).long()
 
     def call(lens):
