@@ -428,14 +428,15 @@ def test_row_map_finds_its_rows(dev, dt):
     assert many <= 2.5 * short
 
 
-def test_spmm_of_few_sorted_rows(dev):
-    """A few thousand rows of unequal length are a wave each, so that the
-    longest, side by side, are not one wave's."""
+@pytest.mark.parametrize("rows,log_mean,k", [(11000, 2.45, 14), (1000, 1, 60)])
+def test_spmm_of_few_sorted_rows(dev, rows, log_mean, k):
+    """A few thousand rows of unequal length are spread over the chip, so that
+    the longest, side by side, are not one wave's."""
     g = torch.Generator().manual_seed(3)
-    lens = torch.exp(1.5 * torch.randn(11000, generator=g) + 2.45)
+    lens = torch.exp(1.5 * torch.randn(rows, generator=g) + log_mean)
     lens = lens.round().clamp(1, 4096).long()
-    G.say("spmm of few sorted rows")
-    mixed = us(_spmm_call(lens, 14, torch.bfloat16, cols=20000))
-    up = us(_spmm_call(lens.sort().values, 14, torch.bfloat16, cols=20000))
+    G.say(f"spmm of {rows} sorted rows k={k}")
+    mixed = us(_spmm_call(lens, k, torch.bfloat16, cols=20000))
+    up = us(_spmm_call(lens.sort().values, k, torch.bfloat16, cols=20000))
     print(f"ascending {up:.1f} us, shuffled {mixed:.1f} us")
     assert up <= 1.6 * mixed

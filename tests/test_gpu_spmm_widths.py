@@ -71,9 +71,16 @@ def test_widths(dev, orc, k, mean, opts, offset, dt):
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 6, 7, 8, 9, 17, 33, 63, 100, 129])
 def test_entries_at_a_time(dev, orc, k, mean, dt):
     """Mean rows on every side of the rule that sets how many entries a row's
-    lanes take at a time, with one row past the group's own steps."""
+    lanes take at a time, with one row past the group's own steps.  The rows
+    fill 2,048 waves, as fewer take more lanes."""
     rng = np.random.default_rng(k)
-    lens = rng.poisson(mean, 901)
+    v = 8 if k >= 8 and dt == torch.bfloat16 else min(4, 1 << (k.bit_length()
+                                                                - 1))
+    lanes = 1
+    while lanes < min(16, -(-k // v)):
+        lanes *= 2
+    at_a_time = 1 if mean < 3 else 2 if mean < 12 else 4 if mean < 48 else 16
+    lens = rng.poisson(mean, 2048 * 64 // min(64, lanes * at_a_time) + 5)
     lens[450] = max(200, lens[450])
     csr = W.csr_from_lengths(rng, lens, 1201)
     rhs = rng.uniform(-1, 1, (csr.cols, k)).astype(np.float32)
